@@ -531,8 +531,12 @@ int resolve(const fpcc_job *job, Dims &d)
 }
 
 // Workspace regions of a job (byte offsets, 256-B aligned).
+// `need` bytes suffice; `total` adds the scratch (at t) that time-domain sums of few
+// rows are split over the chip with.  It is left out where it would take a job past
+// the fixed scratch of fpcc_allpairs_device_noalloc, and unused in a workspace that
+// ends before it.
 struct Layout {
-    size_t a = 0, b = 0, c = 0, d = 0, e = 0, f = 0, total = 0;
+    size_t a = 0, b = 0, c = 0, d = 0, e = 0, f = 0, t = 0, need = 0, total = 0;
 };
 
 bool is_gram(int stack) { return stack == FPCC_STACK_GRAM || stack == FPCC_STACK_GRAM16; }
@@ -544,13 +548,22 @@ size_t take(size_t &total, size_t bytes)
     return off;
 }
 
+Layout add_time_scratch(const fpcc_job *job, const Dims &d, Layout l)
+{
+    l.need = l.t = l.total;
+    if (job->kind != FPCC_PCC1 && job->kind != FPCC_PCCV) return l;
+    const size_t total = l.need + align_up(pcc_time_scratch(d.S, d.W, d.N, d.L, job->stack == FPCC_STACK_NONE ? 0 : 1), 256);
+    if (l.need > FPCC_NOALLOC_SCRATCH_BYTES || total <= FPCC_NOALLOC_SCRATCH_BYTES) l.total = total;
+    return l;
+}
+
 Layout layout(const fpcc_job *job, const Dims &d)
 {
     Layout l;
     const size_t SW = (size_t)d.S * d.W, K1 = d.Nz / 2 + 1;
     if (d.large) {
         l.a = take(l.total, large_workspace(job->kind, job->stack, d.S, d.W, d.N, (int)d.Nz));
-        return l;
+        return add_time_scratch(job, d, l);
     }
     switch (job->kind) {
     case FPCC_PCC2:
@@ -582,12 +595,18 @@ Layout layout(const fpcc_job *job, const Dims &d)
         l.a = take(l.total, wpcc_workspace(d.S, d.W, d.N, (int)d.Nz, (int)d.fam->S));
         break;
     }
-    return l;
+    return add_time_scratch(job, d, l);
 }
 
 }  // namespace
 
 namespace fpcc {
+size_t job_workspace_need(const fpcc_job *job)
+{
+    Dims d;
+    return resolve(job, d) ? 0 : layout(job, d).need;
+}
+
 int job_station_regions(const fpcc_job *job, size_t *off, size_t *per)
 {
     Dims d;
@@ -650,13 +669,14 @@ int station_stage(const fpcc_job *job, const Dims &d, const float *x, char *ws, 
     return -1;
 }
 
-int pair_stage(const fpcc_job *job, const Dims &d, char *ws, float *y, hipStream_t st)
+int pair_stage(const fpcc_job *job, const Dims &d, char *ws, size_t ws_bytes, float *y, hipStream_t st)
 {
     Layout l = layout(job, d);
+    double *part = l.total > l.need && ws_bytes >= l.total ? (double *)(ws + l.t) : nullptr;
     int r = 0;
     if (d.large) {
         const int stack = job->stack == FPCC_STACK_ZSUM ? FPCC_STACK_PLAIN : job->stack;
-        return large_pair_stage(job->kind, stack, d.S, d.W, d.N, (int)d.Nz, d.lag0, d.L, job->v, ws + l.a, y, st);
+        return large_pair_stage(job->kind, stack, d.S, d.W, d.N, (int)d.Nz, d.lag0, d.L, job->v, ws + l.a, y, part, st);
     }
     const int mode = job->stack == FPCC_STACK_NONE ? 0 : 1;
     switch (job->kind) {
@@ -722,7 +742,7 @@ int pair_stage(const fpcc_job *job, const Dims &d, char *ws, float *y, hipStream
     case FPCC_PCC1:
     case FPCC_PCCV:
         return launch_pcc_time((const cf32 *)(ws + l.a), d.S, d.W, d.N, d.lag0, d.L,
-                               job->kind == FPCC_PCC1 ? 1.0 : job->v, job->kind == FPCC_PCC1, mode, y, d.L, 0, st);
+                               job->kind == FPCC_PCC1 ? 1.0 : job->v, job->kind == FPCC_PCC1, mode, y, d.L, 0, part, st);
     case FPCC_WPCC: return wpcc_pair_stage(d.S, d.W, d.N, *d.fam, d.lag0, d.L, mode == 0, ws + l.a, y, st);
     }
     return -1;
@@ -784,9 +804,11 @@ int pcc_time_host(int pcc1, float **y, const float *const *x1, const float *cons
     const size_t bphi = complex_in ? 0
                         : small    ? sizeof(cf32) * 2 * Tr * (size_t)N
                                    : large_workspace(FPCC_PCC1, FPCC_STACK_NONE, 2, (int)Tr, N, N);
+    const size_t tphi = align_up(bphi, 256), bpart = pcc_time_scratch(2, (int)Tr, N, Lp - l1, 0);
     EntryBufs b;
-    if (!b.get(sizeof(float) * xlen, sizeof(float) * ylen, sizeof(float) * xlen, sizeof(float) * ylen, bphi))
+    if (!b.get(sizeof(float) * xlen, sizeof(float) * ylen, sizeof(float) * xlen, sizeof(float) * ylen, tphi + bpart))
         return -1;
+    double *part = bpart ? (double *)((char *)b.dws + tphi) : nullptr;
     int r = upload_rows(
         x1, x2, Tr, (size_t)N * cw, (float *)b.hx, (float *)b.dx,
         [&](unsigned tr) {
@@ -799,7 +821,7 @@ int pcc_time_host(int pcc1, float **y, const float *const *x1, const float *cons
     FPCC_CHECK(hipMemsetAsync(b.dy, 0, sizeof(float) * ylen, nullptr));
     const cf32 *phi;
     if (complex_in) {
-        if ((r = launch_ampnormf_rows((cf32 *)b.dx, 2 * (int)Tr, N, nullptr))) return r;
+        if ((r = launch_half_phasor_rows((cf32 *)b.dx, 2 * (int)Tr, N, nullptr))) return r;
         phi = (const cf32 *)b.dx;
     } else if (small) {
         if ((r = launch_station_phasor((const float *)b.dx, (long long)Tr * N, 2, Tr, N, (cf32 *)b.dws, nullptr)))
@@ -811,7 +833,7 @@ int pcc_time_host(int pcc1, float **y, const float *const *x1, const float *cons
             return r;
         phi = (const cf32 *)b.dws;
     }
-    if ((r = launch_pcc_time(phi, 2, Tr, N, Lag1 + l1, Lp - l1, v, pcc1, 0, (float *)b.dy, L, l1, nullptr)))
+    if ((r = launch_pcc_time(phi, 2, Tr, N, Lag1 + l1, Lp - l1, v, pcc1, 0, (float *)b.dy, L, l1, part, nullptr)))
         return r;
     FPCC_CHECK(hipMemcpy(b.hy, b.dy, sizeof(float) * ylen, hipMemcpyDeviceToHost));
     rows_parallel(Tr, sizeof(float) * ylen, [&](size_t tr) {
@@ -852,7 +874,7 @@ int pair_set_host(int kind, float **y, float **x1, float **x2, unsigned N, unsig
     if (!b.get(sizeof(float) * xlen, sizeof(float) * ylen, sizeof(float) * xlen, sizeof(float) * ylen, wsb)) return -1;
     if ((r = upload_rows(x1, x2, Tr, N, (float *)b.hx, (float *)b.dx, [](unsigned) {}))) return r;
     if ((r = station_stage(&job, d, (const float *)b.dx, (char *)b.dws, nullptr))) return r;
-    if ((r = pair_stage(&job, d, (char *)b.dws, (float *)b.dy, nullptr))) return r;
+    if ((r = pair_stage(&job, d, (char *)b.dws, wsb, (float *)b.dy, nullptr))) return r;
     FPCC_CHECK(hipMemcpy(b.hy, b.dy, sizeof(float) * ylen, hipMemcpyDeviceToHost));
     rows_parallel(Tr, sizeof(float) * (size_t)Tr * d.L,
                   [&](size_t tr) { memcpy(y[tr], (float *)b.hy + tr * d.L, sizeof(float) * d.L); });
@@ -881,7 +903,7 @@ extern "C" int fpcc_station_stage_device(const fpcc_job *job, const float *d_x, 
     Dims d;
     int r = resolve(job, d);
     if (r) return r;
-    if (!d_x || !d_ws || ws_bytes < layout(job, d).total) return -1;
+    if (!d_x || !d_ws || ws_bytes < layout(job, d).need) return -1;
     return station_stage(job, d, d_x, (char *)d_ws, (hipStream_t)stream);
 }
 
@@ -890,8 +912,8 @@ extern "C" int fpcc_pair_stage_device(const fpcc_job *job, void *d_ws, size_t ws
     Dims d;
     int r = resolve(job, d);
     if (r) return r;
-    if (!d_y || !d_ws || ws_bytes < layout(job, d).total) return -1;
-    return pair_stage(job, d, (char *)d_ws, d_y, (hipStream_t)stream);
+    if (!d_y || !d_ws || ws_bytes < layout(job, d).need) return -1;
+    return pair_stage(job, d, (char *)d_ws, ws_bytes, d_y, (hipStream_t)stream);
 }
 
 namespace {
@@ -949,7 +971,7 @@ extern "C" int fpcc_pair_stage_batch_device(const fpcc_job *jobs, int njobs, voi
     for (int j = 0; j < njobs; ++j) {
         int r = resolve(&jobs[j], D[j]);
         if (r) return r;
-        if (!d_ws[j] || !d_y[j] || ws_bytes[j] < layout(&jobs[j], D[j]).total) return -1;
+        if (!d_ws[j] || !d_y[j] || ws_bytes[j] < layout(&jobs[j], D[j]).need) return -1;
         int m;
         if (pair_batch_mode(&jobs[j], D[j], m)) {
             mode[j] = m;
@@ -966,7 +988,7 @@ extern "C" int fpcc_pair_stage_batch_device(const fpcc_job *jobs, int njobs, voi
         for (int g : grp) done[g] = 1;
         int r;
         if (grp.size() == 1) {
-            r = pair_stage(&jobs[i], D[i], (char *)d_ws[i], d_y[i], st);
+            r = pair_stage(&jobs[i], D[i], (char *)d_ws[i], ws_bytes[i], d_y[i], st);
         } else if (jobs[i].kind != FPCC_PCC2) {
             const bool gn = jobs[i].kind == FPCC_GNCC;
             GnBatch jb{};
@@ -1176,7 +1198,7 @@ extern "C" int fpcc_station_stage_batch_device(const fpcc_job *jobs, int njobs, 
     for (int j = 0; j < njobs; ++j) {
         int r = resolve(&jobs[j], D[j]);
         if (r) return r;
-        if (!d_x[j] || !d_ws[j] || ws_bytes[j] < layout(&jobs[j], D[j]).total) return -1;
+        if (!d_x[j] || !d_ws[j] || ws_bytes[j] < layout(&jobs[j], D[j]).need) return -1;
     }
     std::vector<char> done(njobs, 0);
     for (int i = 0; i < njobs; ++i) {

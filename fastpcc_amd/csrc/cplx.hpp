@@ -31,6 +31,17 @@ template <int DIR, typename R> __host__ __device__ __forceinline__ C2<R> rot(C2<
 {
     return DIR < 0 ? C2<R>{a.y, -a.x} : C2<R>{-a.y, a.x};
 }
+// The half-angle phasor alpha of an analytic sample z: alpha^2 = z / (|z| + eps)
+// (AmpNormf's factor in FP32; 0 where it is not normal), the principal root,
+// formed in FP64 and rounded once.
+__device__ __forceinline__ cf32 half_phasor(cf32 z, float eps)
+{
+    const float r = 1.0f / (sqrtf(z.x * z.x + z.y * z.y) + eps);
+    if (!__builtin_isnormal(r) || (z.x == 0.0f && z.y == 0.0f)) return cf32{0.0f, 0.0f};
+    const double x = z.x, y = z.y, a = sqrt(x * x + y * y);
+    const double big = sqrt(0.5 * (double)r * (a + fabs(x))), small = 0.5 * (double)r * fabs(y) / big;
+    return z.x >= 0.0f ? cf32{(float)big, (float)copysign(small, y)} : cf32{(float)small, (float)copysign(big, y)};
+}
 template <typename R> __host__ __device__ __forceinline__ R norm2(C2<R> a) { return a.x * a.x + a.y * a.y; }
 
 // ---- compile-time cos/sin of 2*pi*num/den (Taylor series on [-pi, pi]) ----

@@ -9,15 +9,18 @@ namespace fpcc {
 // PCC2 station stage: F[s*W+w][Nz] = FFT_Nz(pad(AmpNormf(analytic_N(x_sw))))
 int launch_station_pcc(const float *d_x, long long station_stride, int S, int W, int N, int Nz, cf32 *d_F,
                        hipStream_t st);
-// AmpNormf in place on `rows` rows of N complex values.
-int launch_ampnormf_rows(cf32 *d_z, int rows, int N, hipStream_t st);
-// Phasors only (analytic signal + AmpNormf), phi[s*W+w][N].
+// Half-angle phasors (pcc_time.hip) in place of `rows` rows of N analytic samples.
+int launch_half_phasor_rows(cf32 *d_z, int rows, int N, hipStream_t st);
+// Half-angle phasors only (analytic signal + AmpNormf, pcc_time.hip), phi[s*W+w][N].
 int launch_station_phasor(const float *d_x, long long station_stride, int S, int W, int N, cf32 *d_phi,
                           hipStream_t st);
-// Time-domain PCC1 (pcc1 = 1) or PCC-v over lags lag_first .. lag_first+L-1;
+// Time-domain PCC1 (pcc1 = 1) or PCC-v of half-angle phasors over lags lag_first .. lag_first+L-1;
 // output element l of row r at y[r*out_ld + out_off + l] (rows: pair*W+w or pair).
 int launch_pcc_time(const cf32 *d_phi, int S, int W, int N, int lag_first, int L, double v, int pcc1, int mode,
-                    float *d_y, int out_ld, int out_off, hipStream_t st);
+                    float *d_y, int out_ld, int out_off, double *part, hipStream_t st);
+// bytes of `part` (partial sums of a split launch; 0: not split).  launch_pcc_time
+// with part == nullptr runs unsplit.
+size_t pcc_time_scratch(int S, int W, int N, int L, int mode);
 // PCC2 pair stage over pairs [pair_base, pair_base+npairs) of S stations.
 // mode 0: y[p][w][L]; 1: mean over windows of per-window IFFTs; 2: IFFT of the
 // window sum (same result by linearity).
@@ -182,7 +185,7 @@ int large_station_stage(int kind, const float *x, long long stride, int S, int W
 int large_pcc2_station_batch(int n, const float *const *x, const long long *stride, const int *S, const int *W,
                              const int *N, const int *stack, int Nz, char *const *ws, hipStream_t st);
 int large_pair_stage(int kind, int stack, int S, int W, int N, int Nz, int lag0, int L, double v, char *ws, float *y,
-                     hipStream_t st);
+                     double *part, hipStream_t st);
 // Workspace regions holding the station stage's per-station output (what the pair
 // stage reads): station s at off[k] + s*per[k]; returns the region count.
 int large_station_regions(int kind, int stack, int S, int W, int N, int Nz, size_t *off, size_t *per);
@@ -215,6 +218,9 @@ int wpcc_pair_stage(int S, int W, int N, const WFamily &f, int lag0, int L, bool
 // station's rows are the same in any job with the same kind, windows, N and Nz
 // (and, for WPCC, filter parameters).
 int job_station_regions(const fpcc_job *job, size_t *off, size_t *per);
+// Bytes of workspace a job runs in (0 if invalid): fpcc_workspace_size without the
+// optional scratch of split time-domain sums.
+size_t job_workspace_need(const fpcc_job *job);
 // Whether the job's station stage can share launches with other jobs of the same
 // key (fpcc_station_stage_batch_device).
 bool job_batch_key(const fpcc_job *job, long long *key);

@@ -6,7 +6,7 @@
 //   mask and both row passes fused; any other N: Bluestein chirp convolutions on a
 //   power-of-two grid), max|z|^2 per window, AmpNormf and zero pad
 //   fused into the first pass of FFT_Nz; spectra stay in permuted bin order.
-// PCC1 / PCC-v: the same analytic signal, AmpNormf per row, then the time-domain kernel.
+// PCC1 / PCC-v: the same analytic signal, half-angle phasors per row, then the time-domain kernel.
 // GNCC / 1-bit: complex FFT_Nz of the zero-padded samples (or signs); energies as
 //   FP64 prefix sums.  (GNCC runs its large-N FFTs in FP32.)
 // Pair stage: inverse row pass with the cross spectrum conj(F_i) F_j (summed over
@@ -297,7 +297,7 @@ int large_station_stage(int kind, const float *x, long long stride, int S, int W
     case FPCC_PCCV: {
         cf32 *Z = (cf32 *)(ws + l.Z);
         if ((r = analytic_big(x, stride, S, W, N, Z, (float *)(ws + l.mx), (cf32 *)(ws + l.B), st))) return r;
-        return launch_ampnormf_rows(Z, SW, N, st);
+        return launch_half_phasor_rows(Z, SW, N, st);
     }
     case FPCC_GNCC:
     case FPCC_CC1B: {
@@ -363,7 +363,7 @@ int large_pcc2_station_batch(int n, const float *const *x, const long long *stri
 }
 
 int large_pair_stage(int kind, int stack, int S, int W, int N, int Nz, int lag0, int L, double v, char *ws, float *y,
-                     hipStream_t st)
+                     double *part, hipStream_t st)
 {
     LargeLayout l = large_layout(kind, stack, S, W, N, Nz);
     const int P = S * (S - 1) / 2;
@@ -371,7 +371,7 @@ int large_pair_stage(int kind, int stack, int S, int W, int N, int Nz, int lag0,
     if (kind == FPCC_PCC1 || kind == FPCC_PCCV) {
         const int mode = stack == FPCC_STACK_NONE ? 0 : 1;
         return launch_pcc_time((const cf32 *)(ws + l.Z), S, W, N, lag0, L, kind == FPCC_PCC1 ? 1.0 : v,
-                               kind == FPCC_PCC1, mode, y, L, 0, st);
+                               kind == FPCC_PCC1, mode, y, L, 0, part, st);
     }
     const BigPlan &bz = big_plan(Nz);
     // scale and normalisation of each type (pcc2_set :832, ccf/cc_lowlevel 1/Nz, gn(f)_lowlevel)

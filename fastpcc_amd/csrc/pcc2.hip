@@ -23,7 +23,7 @@
 namespace fpcc {
 
 // One station-window: analytic signal, AmpNormf, zero-padding to Nz and FFT_Nz
-// into Frow (or, phirow != nullptr, the length-N phasors).
+// into Frow (or, phirow != nullptr, the length-N half-angle phasors).
 __device__ void station_pcc_row(const float *__restrict__ in, int N, int Nz, const FftPlan &planN,
                                 const cf32 *__restrict__ twN, const FftPlan &planZ, const cf32 *__restrict__ twZ,
                                 float da1, cf32 *__restrict__ Frow, cf32 *__restrict__ phirow,
@@ -61,12 +61,8 @@ __device__ void station_pcc_row(const float *__restrict__ in, int N, int Nz, con
     }
     m = block_max(m, red);
     const float eps = (float)(1e-6 * sqrt((double)m));
-    if (phirow) {  // phasor-only output (time-domain PCC1 / PCC-v)
-        for (int n = threadIdx.x; n < N; n += T) {
-            cf32 v = z[n];
-            float r = 1.0f / (sqrtf(v.x * v.x + v.y * v.y) + eps);
-            phirow[n] = __builtin_isnormal(r) ? cf32{v.x * r, v.y * r} : cf32{0.0f, 0.0f};
-        }
+    if (phirow) {  // half-angle phasors only (time-domain PCC1 / PCC-v)
+        for (int n = threadIdx.x; n < N; n += T) phirow[n] = half_phasor(z[n], eps);
         return;
     }
     cf32 *dst = (z == buf0) ? buf1 : buf0;
@@ -234,8 +230,9 @@ k_station_pcc_3600(const float *__restrict__ x, long long station_stride, int W,
     for (int i = 0; i < kSpM / kSpT; ++i) out[t + kSpT * i] = float4{ev[i].x, ev[i].y, v[i].x, v[i].y};
 }
 
-// AmpNormf (src/FFTapps.c:178-205) in place on rows of N complex values.
-__global__ void __launch_bounds__(256) k_ampnormf_rows(cf32 *__restrict__ z, int N)
+// AmpNormf (src/FFTapps.c:178-205) on rows of N analytic samples, in place, as
+// half-angle phasors (pcc_time.hip).
+__global__ void __launch_bounds__(256) k_half_phasor_rows(cf32 *__restrict__ z, int N)
 {
     __shared__ float red[4];
     cf32 *row = z + (long long)blockIdx.x * N;
@@ -246,11 +243,7 @@ __global__ void __launch_bounds__(256) k_ampnormf_rows(cf32 *__restrict__ z, int
     }
     m = block_max(m, red);
     const float eps = (float)(1e-6 * sqrt((double)m));
-    for (int n = threadIdx.x; n < N; n += blockDim.x) {
-        cf32 v = row[n];
-        float r = 1.0f / (sqrtf(v.x * v.x + v.y * v.y) + eps);
-        row[n] = __builtin_isnormal(r) ? cf32{v.x * r, v.y * r} : cf32{0.0f, 0.0f};
-    }
+    for (int n = threadIdx.x; n < N; n += blockDim.x) row[n] = half_phasor(row[n], eps);
 }
 
 // Fold conj(F1)F2 into the half-length spectrum Z (see file header) in LDS.
@@ -461,11 +454,11 @@ int launch_pair_pcc2(const cf32 *d_F, int S, int W, int N, int Nz, int lag0, int
 }  // namespace fpcc
 
 namespace fpcc {
-int launch_ampnormf_rows(cf32 *d_z, int rows, int N, hipStream_t st)
+int launch_half_phasor_rows(cf32 *d_z, int rows, int N, hipStream_t st)
 {
     if (rows <= 0) return 0;
-    ProfScope prof("ampnormf_rows", st);
-    hipLaunchKernelGGL(k_ampnormf_rows, dim3(rows), dim3(256), 0, st, d_z, N);
+    ProfScope prof("half_phasor_rows", st);
+    hipLaunchKernelGGL(k_half_phasor_rows, dim3(rows), dim3(256), 0, st, d_z, N);
     FPCC_CHECK(hipGetLastError());
     return 0;
 }

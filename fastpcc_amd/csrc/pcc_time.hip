@@ -5,13 +5,29 @@
 // x2 first, src/FFTapps.c:598, :735):
 //   PCC1:  y = sum(|a+b| - |a-b|) / (2 count)               (sqrtf terms)
 //   PCC-v: y = sum(|a+b|^v - |a-b|^v) / (2^(v/2) count)     (powf(|.|^2, v/2) terms)
-// FP32 terms; per 256-sample tile an FP32 partial sum, accumulated in double
-// across tiles (the reference accumulates every term in double).
 //
-// Workgroup: 256 consecutive lags of one pair (one thread per lag) over one
-// window (per-window output) or all windows (mean).  Each 256-sample tile of
-// phi1 and the matching 511 samples of phi2 are staged in LDS; phi1[n] is read
-// by the whole wave at once (broadcast).
+// The station stage keeps the half-angle phasors alpha, alpha^2 = a (half_phasor,
+// cplx.hpp).  With alpha conj(beta) = p + i q and d = |alpha|^2 - |beta|^2,
+//   |a + b|^2 = 4 p^2 + d^2,   |a - b|^2 = 4 q^2 + d^2
+// are sums of squares: no cancellation where a is close to -b or to b (the identity
+// through 2 Re(a conj b) loses the terms there).  P = 2p and Q = 2q are products of
+// rank 2 of the samples of a row and a column, so a 32 x 32 tile (i, j) of terms is two
+// MFMAs.  FP32 MFMAs take the vector unit's own multipliers (measured: 2 ns each a wave
+// of terms on top of the terms), bf16 ones run beside it (0.3 ns): every component is
+// split into three bf16 parts (24 bits, exact) and the products of two components
+// except lowest x lowest (2^-32) fill K = 16.
+//
+// PCC1 needs |a+b| - |a-b| = |P| - |Q| + (corr(P) - corr(Q)), 0 <= corr(x) =
+// sqrt(x^2 + d^2) - |x| <= d^2 / (2|x|).  Square roots run at a quarter of the vector
+// rate, so groups of four terms a lane first test that corr <= 2^-24, FP32's rounding
+// of a term (|a+b| <= 2), throughout the wave, with a bound of |d| over the group's
+// rows; only groups that fail take the roots.  d is the difference of two
+// regularisers 1e-6 max|z| / |z|: 1e-5 in noise, where 1 in 10 groups fails; windows
+// with an event 30 times the noise fail mostly and run no slower than the roots alone.
+// 16 stations x 24 windows of 3600, 2001 lags: 9.40 ms with 12 vector operations a term
+// (sums, differences and squares formed term by term), 5.21 ms here, bound by the
+// vector unit (84% busy, about 7 operations a term).
+#include <algorithm>
 #include "engine.hpp"
 #include "kernels.hpp"
 #include "profile.hpp"
@@ -19,10 +35,6 @@
 
 namespace fpcc {
 
-constexpr int kPtLags = 256;
-constexpr int kPtTile = 256;
-
-// y rows start at out_off within rows of out_ld floats.
 // Hardware square root and power (v_sqrt_f32; v_log_f32 and v_exp_f32, i.e.
 // 2^(V log2 x)), about 1 ulp and a few ulp per term, as the reference's CUDA
 // engine compiles its terms (fast math); the correctly rounded library versions
@@ -34,110 +46,430 @@ __device__ __forceinline__ float hw_pow(float x, float V)
     return __builtin_amdgcn_exp2f(V * __builtin_amdgcn_logf(x));
 }
 
-__global__ void __launch_bounds__(kPtLags)
-k_pcc_time(const cf32 *__restrict__ phi, int S, int W, int N, int lag_first, int L, int pcc1, float V,
-           double div_pow, int mode, float *__restrict__ y, int out_ld, int out_off)
+typedef float f16v __attribute__((ext_vector_type(16)));
+typedef __bf16 b8v __attribute__((ext_vector_type(8)));
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef unsigned u4v __attribute__((ext_vector_type(4)));
+
+enum { PT_SQRT = 0, PT_SQUARE = 1, PT_HWPOW = 2, PT_POW = 3 };
+
+constexpr float kPtD = 2896.3093757400986f;  // (2^11.5 d)^2 <= |x|: corr(x) <= 2^-24
+
+// A component's 8 K slots from its bf16 parts h + m + l, each the rounded rest: left
+// (h h m m h l m l) against right (h m h m l h l m)
+__device__ __forceinline__ unsigned round_bf16(float v)  // in the upper half
 {
-    __shared__ cf32 s1[kPtTile];
-    __shared__ cf32 s2[kPtTile + kPtLags - 1];
-    const int lb = blockIdx.x;
-    int p, w0, w1;
+    const unsigned u = __float_as_uint(v);
+    return (u + 0x7fffu + ((u >> 16) & 1u)) & 0xffff0000u;
+}
+__device__ __forceinline__ void split3(float v, unsigned &h, unsigned &m, unsigned &l)
+{
+    h = round_bf16(v);
+    const float r = v - __uint_as_float(h);
+    m = round_bf16(r);
+    l = __float_as_uint(r - __uint_as_float(m));  // at most 8 bits are left
+}
+// the upper halves of a (low) and b (high)
+__device__ __forceinline__ unsigned pack_hi(unsigned a, unsigned b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
+__device__ __forceinline__ u4v slots_left(float v)
+{
+    unsigned h, m, l;
+    split3(v, h, m, l);
+    return u4v{pack_hi(h, h), pack_hi(m, m), pack_hi(h, l), pack_hi(m, l)};
+}
+__device__ __forceinline__ u4v slots_right(float v)
+{
+    unsigned h, m, l;
+    split3(v, h, m, l);
+    const unsigned hm = pack_hi(h, m);
+    return u4v{hm, hm, pack_hi(l, h), pack_hi(l, m)};
+}
+// 1 - |alpha|^2, and a bound of |1 - |alpha|^2| such that the difference of two is at
+// most the larger bound, times 2^11.5; one that lets no group pass where the bound is
+// past 0.8 or the magnitude past 1 by more than rounding (records near FP32's smallest
+// squares)
+__device__ __forceinline__ float pt_delta(cf32 v) { return (float)(1.0 - ((double)v.x * v.x + (double)v.y * v.y)); }
+__device__ __forceinline__ float pt_bound(float delta)
+{
+    const float b = kPtD * (delta + 1.2e-7f);
+    return delta < -1.2e-7f || b > 0.8f ? 1e6f : b;
+}
+
+// The 16 terms of a lane, added to acc.  db: delta of the lane's column, bb its bound;
+// rd: deltas of the tile's rows, rb the bounds' maxima over runs of 8 rows, in LDS
+// (lane rows 8 g + 4 h + r, g, r < 4).
+template <int FN>
+__device__ __forceinline__ void pt_tile(float (&acc)[16], f16v P, f16v Q, float db, float bb, const float *rd,
+                                        const float *rb, int h, float V)
+{
+    if constexpr (FN == PT_SQUARE) {  // |a+b|^2 - |a-b|^2: d cancels
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] = fmaf(-Q[r], Q[r], fmaf(P[r], P[r], acc[r]));
+        return;
+    }
+    const auto roots = [&](int g) {  // P, Q of group g as |a+b|^v, |a-b|^v
+        const f4v da = *reinterpret_cast<const f4v *>(rd + 8 * g + 4 * h);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int r = 4 * g + e;
+            const float d = da[e] - db, dd = d * d, s = fmaf(P[r], P[r], dd), u = fmaf(Q[r], Q[r], dd);
+            if constexpr (FN == PT_SQRT) {
+                P[r] = hw_sqrt(s);
+                Q[r] = hw_sqrt(u);
+            } else if constexpr (FN == PT_HWPOW) {
+                P[r] = hw_pow(s, V);
+                Q[r] = hw_pow(u, V);
+            } else {
+                P[r] = powf(s, V);
+                Q[r] = powf(u, V);
+            }
+        }
+    };
+    if constexpr (FN == PT_SQRT) {
+        // min(|P|, |Q|) >= tau, tau = b^2 for the larger bound b = 2^11.5 B, follows from
+        // ||P| - |Q|| <= 2 - 2B - 1.3 tau: P^2 + Q^2 = 4 |alpha beta|^2 >= 4 (1 - B)^2, and
+        // sqrt(4 rho^2 - m^2) - m falls with m; 1e-6 for the rounding of the difference
+        const f4v ra = *reinterpret_cast<const f4v *>(rb);
+        float f[4], z[16];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            float m = 0.0f;
+#pragma unroll
+            for (int r = 4 * g; r < 4 * g + 4; ++r) {
+                z[r] = fabsf(P[r]) - fabsf(Q[r]);
+                m = fmaxf(m, fabsf(z[r]));
+            }
+            const float b = fmaxf(ra[g], bb);
+            f[g] = fmaf(b, fmaf(1.3f, b, 2.0f / kPtD), m);
+        }
+        const float fm = fmaxf(fmaxf(f[0], f[1]), fmaxf(f[2], f[3]));
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(fm > 2.0f - 1e-6f) != 0, 0)) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                if (__builtin_amdgcn_ballot_w64(f[g] > 2.0f - 1e-6f) == 0) continue;
+                roots(g);
+#pragma unroll
+                for (int r = 4 * g; r < 4 * g + 4; ++r) z[r] = P[r] - Q[r];
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] += z[r];
+        return;
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) roots(g);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = acc[r] + P[r] - Q[r];
+}
+
+constexpr int kPtWaves = 4;
+constexpr int kPtChunk = 512;  // samples staged at a time
+constexpr int kPtFlush = 4;    // chunks (16 terms a lane and tile each) summed in FP32 before FP64
+
+__host__ __device__ constexpr int pt_bands(int tpw) { return kPtWaves * tpw - 1; }  // 32-lag bands a workgroup
+
+// How the terms of one output row (a pair-window, or a pair whose rw windows are
+// averaged) are spread: G units, each a run of windows, or (ns > 1) one of ns equal
+// parts of one window's samples.
+struct PtSplit {
+    int G, ns, nblk;  // units a row, parts a window, lag blocks a row
+};
+
+// Workgroup of 4 waves: one lag block of 32 (4 TPW - 1) lags of one unit.  Tile c
+// (wave c mod 4) is the square of terms (m, n) = (n0 + lagA + 32 c + i, n0 + j),
+// i, j < 32, walked down the diagonal n0 = nstart, nstart + 32, ...: its sums over
+// i - j = r belong to lag lagA + 32 c + r, so 4 TPW tiles cover 4 TPW - 1 bands of 32
+// lags.  Each chunk of samples is staged in LDS by components (out-of-range samples
+// as alpha = 0, whose terms are zero).  The 16 FP32 sums a lane are added along the
+// tile's diagonals in FP64 every 4 chunks (64 terms).
+// Two or three waves a SIMD asked for: within 256 registers the MFMA results land in
+// ordinary registers (else the compiler puts them in accumulation registers, three
+// more moves a term).
+// MFMA 32x32x16 layout: lane l holds A[l%32][8 (l/32) ..], B[8 (l/32) ..][l%32] and
+// D[8 (r/4) + 4 (l/32) + r%4][l%32], r < 16; its half-wave holds the slots of one
+// component: P (ax | ay)(2bx | 2by), Q (ax | ay)(-2by | 2bx).
+template <int FN, int TPW>
+__global__ void __launch_bounds__(64 * kPtWaves) __attribute__((amdgpu_waves_per_eu(TPW == 4 ? 2 : 3)))
+k_pcc_time(const cf32 *__restrict__ phi, int S, int W, int N, int lag_first, int L, float V, double div, int mode,
+           PtSplit sp, float *__restrict__ y, int out_ld, int out_off, double *__restrict__ part)
+{
+    constexpr int kT = 64 * kPtWaves, kTiles = kPtWaves * TPW, kA = kPtChunk + 32 * (kTiles - 1);
+    __shared__ u4v bc[3][kPtChunk], ac[2][kA];                  // 2bx, 2by, -2by; ax, ay
+    __shared__ __align__(16) float bd[kPtChunk], ad[kA], ab[kA / 8];  // deltas; the rows' bounds by 8
+    // between chunks the operands' space serves the sums along diagonals
+    float (*tile)[32 * 33] = reinterpret_cast<float (*)[32 * 33]>(ac);
+    double (*diag)[64] = reinterpret_cast<double (*)[64]>(bc);
+    static_assert(sizeof(float) * kPtWaves * 32 * 33 <= sizeof(ac) && sizeof(double) * kTiles * 64 <= sizeof(bc), "fit");
+    const int t = threadIdx.x, lane = t & 63, h = lane >> 5, lj = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int lb = blockIdx.x % sp.nblk;
+    const int ru = blockIdx.x / sp.nblk, u = ru % sp.G, row = ru / sp.G;
+    const int p = mode == 0 ? row / W : row;
+    // windows and sample range of this unit
+    int w0, w1, part_i = 0;
     if (mode == 0) {
-        p = blockIdx.y / W;
-        w0 = blockIdx.y % W;
+        w0 = row - p * W;
         w1 = w0 + 1;
+        part_i = u;
+    } else if (sp.ns > 1) {
+        w0 = u / sp.ns;
+        w1 = w0 + 1;
+        part_i = u - w0 * sp.ns;
     } else {
-        p = blockIdx.y;
-        w0 = 0;
-        w1 = W;
+        w0 = (int)((long long)u * W / sp.G);
+        w1 = (int)((long long)(u + 1) * W / sp.G);
     }
     int i, j;
     pair_index(p, S, i, j);
-    const int tid = threadIdx.x;
-    const int lagA = lag_first + lb * kPtLags;
-    const int lagB = min(lagA + kPtLags - 1, lag_first + L - 1);
-    const int lag = lagA + tid;
-    const bool valid = lag <= lagB;
-    const int n_lo = max(0, -lag), n_hi = min(N, N - lag);
-    const int nstart = max(0, -lagB), nend = min(N, N - lagA);
-    float mean = 0.0f;
+    const int lagA = lag_first + lb * 32 * pt_bands(TPW);
+    const int lagB = min(lagA + 32 * pt_bands(TPW) - 1, lag_first + L - 1);
+    const int Lb = lagB - lagA + 1;
+    int nstart = max(0, -lagB), nend = min(N, N - lagA);
+    if (sp.ns > 1) {
+        const int per = ((nend - nstart + sp.ns - 1) / sp.ns + 31) / 32 * 32;
+        nstart += part_i * per;
+        nend = min(nend, nstart + per);
+    }
+    const u4v *bp = bc[h] + lj, *bq = bc[h ? 0 : 2] + lj, *ap = ac[h] + lj;  // by half-wave
+
+    float acc[TPW][16];
+    double dsum[TPW];  // lane l < 63: the tile's diagonal r = l - 31
+#pragma unroll
+    for (int k = 0; k < TPW; ++k) {
+        dsum[k] = 0.0;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[k][r] = 0.f;
+    }
+    auto flush = [&]() {
+        float *sc = tile[wave];
+#pragma unroll
+        for (int k = 0; k < TPW; ++k) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                sc[(8 * (r >> 2) + 4 * h + (r & 3)) * 33 + lj] = acc[k][r];
+                acc[k][r] = 0.f;
+            }
+            // the scratch is the wave's own: its writes land before its reads
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
+            const int r = lane - 31;
+#pragma unroll 8
+            for (int jj = 0; jj < 32; ++jj) {
+                const int ii = jj + r;
+                if (ii >= 0 && ii < 32) dsum[k] += (double)sc[ii * 33 + jj];
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
+        }
+    };
+    int chunks = 0;
     for (int w = w0; w < w1; ++w) {
         const cf32 *p1 = phi + (long long)(i * W + w) * N;
         const cf32 *p2 = phi + (long long)(j * W + w) * N;
-        double acc = 0.0;
-        for (int n0 = nstart; n0 < nend; n0 += kPtTile) {
-            __syncthreads();
-            for (int t = tid; t < kPtTile; t += kPtLags) {
-                const int n = n0 + t;
-                s1[t] = (n < N) ? p1[n] : cf32{0.f, 0.f};
+        cf32 fb[kPtChunk / kT], fa[(kA + kT - 1) / kT];  // the next chunk's samples, loaded ahead
+        auto fetch = [&](int n0) {
+#pragma unroll
+            for (int i = 0; i < kPtChunk / kT; ++i) {
+                const int n = n0 + t + kT * i;
+                fb[i] = n < nend ? p1[n] : cf32{0.f, 0.f};
             }
-            for (int t = tid; t < kPtTile + kPtLags - 1; t += kPtLags) {
-                const int m = n0 + lagA + t;
-                s2[t] = (m >= 0 && m < N) ? p2[m] : cf32{0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < (kA + kT - 1) / kT; ++i) {
+                const int m = n0 + lagA + t + kT * i;
+                fa[i] = m >= 0 && m < N ? p2[m] : cf32{0.f, 0.f};
             }
+        };
+        fetch(nstart);
+        for (int n0 = nstart; n0 < nend; n0 += kPtChunk) {
             __syncthreads();
-            if (!valid) continue;
-            const int lo = max(n_lo, n0) - n0, hi = min(n_hi, n0 + kPtTile) - n0;
-            float part = 0.0f;
-            // full tiles (the common case) as a fixed-count loop the compiler
-            // unrolls, so the LDS reads of several terms are in flight together
-            auto run = [&](auto term) {
-                if (lo == 0 && hi == kPtTile) {
-#pragma unroll 16
-                    for (int t = 0; t < kPtTile; ++t) part += term(s2[t + tid], s1[t]);
-                } else {
-                    for (int t = lo; t < hi; ++t) part += term(s2[t + tid], s1[t]);
+#pragma unroll
+            for (int i = 0; i < kPtChunk / kT; ++i) {
+                const int e = t + kT * i;
+                const u4v sy = slots_right(2 * fb[i].y);
+                bc[0][e] = slots_right(2 * fb[i].x);
+                bc[1][e] = sy;
+                bc[2][e] = sy ^ 0x80008000u;
+                bd[e] = pt_delta(fb[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < (kA + kT - 1) / kT; ++i) {
+                const int e = t + kT * i;
+                const float d = pt_delta(fa[i]);
+                // the maximum over 8 samples: 8 lanes
+                float b = pt_bound(d);
+                b = fmaxf(b, __shfl_xor(b, 1, 64));
+                b = fmaxf(b, __shfl_xor(b, 2, 64));
+                b = fmaxf(b, __shfl_xor(b, 4, 64));
+                if (e < kA) {
+                    ac[0][e] = slots_left(fa[i].x);
+                    ac[1][e] = slots_left(fa[i].y);
+                    ad[e] = d;
+                    if ((e & 7) == 0) ab[e >> 3] = b;
                 }
-            };
-            // PCC1, and PCC-v at v = 1 (|.|^2 to the power 1/2), take square roots; PCC-v
-            // at v = 2 takes the squared magnitudes themselves (powf(x, 1) = x)
-            if (pcc1 || V == 0.5f) {
-                run([](cf32 a, cf32 b) {
-                    const float sx = a.x + b.x, sy = a.y + b.y, dx = a.x - b.x, dy = a.y - b.y;
-                    return hw_sqrt(sx * sx + sy * sy) - hw_sqrt(dx * dx + dy * dy);
-                });
-            } else if (V == 1.0f) {
-                run([](cf32 a, cf32 b) {
-                    const float sx = a.x + b.x, sy = a.y + b.y, dx = a.x - b.x, dy = a.y - b.y;
-                    return (sx * sx + sy * sy) - (dx * dx + dy * dy);
-                });
-            } else if (V > 0.f) {
-                run([V](cf32 a, cf32 b) {
-                    const float sx = a.x + b.x, sy = a.y + b.y, dx = a.x - b.x, dy = a.y - b.y;
-                    return hw_pow(sx * sx + sy * sy, V) - hw_pow(dx * dx + dy * dy, V);
-                });
-            } else {
-                run([V](cf32 a, cf32 b) {
-                    const float sx = a.x + b.x, sy = a.y + b.y, dx = a.x - b.x, dy = a.y - b.y;
-                    return powf(sx * sx + sy * sy, V) - powf(dx * dx + dy * dy, V);
-                });
             }
-            acc += (double)part;
-        }
-        const int count = n_hi - n_lo;
-        float v;
-        if (pcc1) v = (float)acc / (float)(2 * count);  // src/FFTapps.c:276
-        else v = (float)(acc / (div_pow * count));      // :334
-        if (mode == 0) {
-            if (valid) y[((long long)p * W + w) * out_ld + out_off + lb * kPtLags + tid] = v;
-        } else {
-            mean += v;
+            __syncthreads();
+            if (n0 + kPtChunk < nend) fetch(n0 + kPtChunk);
+            // tiles of all steps in one sequence, software-pipelined: the operands of the
+            // tile after next load and the next tile's MFMAs run while a tile's terms are
+            // summed (its results in the other half of P, Q)
+            const int nst = min(kPtChunk, nend - n0);
+            f16v P[2], Q[2];
+            u4v b_p = bp[0], b_q = bq[0], a_p = ap[32 * wave];
+            auto mfma = [&](int x) {
+                const f16v z = {};
+                P[x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(b8v, a_p), __builtin_bit_cast(b8v, b_p), z, 0, 0, 0);
+                Q[x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(b8v, a_p), __builtin_bit_cast(b8v, b_q), z, 0, 0, 0);
+            };
+            // operands of tile k of the step at n (a wave's tiles are c = wave, wave + 4, ...);
+            // past the last step they are loaded, not used
+            auto load = [&](int n, int k) {
+                const int nb = min(n, kPtChunk - 32);
+                if (k == 0) {
+                    b_p = bp[nb];
+                    b_q = bq[nb];
+                }
+                a_p = ap[nb + 32 * (wave + kPtWaves * k)];
+            };
+            mfma(0);
+            load(0, 1);
+            for (int n = 0; n < nst; n += 32) {
+                const float db = bd[n + lj], bb = pt_bound(db);
+#pragma unroll
+                for (int k = 0; k < TPW; ++k) {
+                    mfma((k + 1) & 1);
+                    load(k + 2 < TPW ? n : n + 32, (k + 2) % TPW);
+                    const int e0 = n + 32 * (wave + kPtWaves * k), m0 = n0 + lagA + e0;
+                    // tiles of no lag of this block, or outside the other window, hold no terms
+                    if (32 * (wave + kPtWaves * k) - 31 < Lb && m0 + 31 >= 0 && m0 < N)
+                        pt_tile<FN>(acc[k], P[k & 1], Q[k & 1], db, bb, ad + e0, ab + e0 / 8, h, V);
+                }
+            }
+            if (++chunks == kPtFlush) {
+                chunks = 0;
+                __syncthreads();
+                flush();
+            }
         }
     }
-    if (mode != 0 && valid) y[(long long)p * out_ld + out_off + lb * kPtLags + tid] = mean / (float)W;
+    __syncthreads();
+    if (chunks) flush();
+#pragma unroll
+    for (int k = 0; k < TPW; ++k) diag[wave + kPtWaves * k][lane] = dsum[k];
+    __syncthreads();
+    // lag lagA + 32 c + r: diagonal r of tile c and diagonal r - 32 of tile c + 1
+    for (int l = t; l < Lb; l += kT) {
+        const int c = l >> 5, r = l & 31;
+        const double sum = diag[c][31 + r] + (r ? diag[c + 1][r - 1] : 0.0);
+        const int gl = lb * 32 * pt_bands(TPW) + l;
+        if (sp.G > 1) {
+            part[(long long)ru * L + gl] = sum;
+        } else {
+            const int lag = lagA + l, count = max(0, min(N, N - lag) - max(0, -lag));
+            y[(long long)row * out_ld + out_off + gl] = (float)(sum / (div * count));
+        }
+    }
+}
+
+// The G partial sums of every lag of a row, in order, normalised.
+__global__ void __launch_bounds__(256)
+k_pcc_time_sum(const double *__restrict__ part, int N, int lag_first, int L, int G, double div, float *__restrict__ y,
+               int out_ld, int out_off)
+{
+    const int l = blockIdx.x * 256 + threadIdx.x;
+    const long long row = blockIdx.y;  // G > 1 only where rows are few
+    if (l >= L) return;
+    double sum = 0.0;
+    for (int u = 0; u < G; ++u) sum += part[(row * G + u) * L + l];
+    const int lag = lag_first + l, count = max(0, min(N, N - lag) - max(0, -lag));
+    y[row * out_ld + out_off + l] = (float)(sum / (div * count));
+}
+
+namespace {
+
+// Lag blocks and units of a launch (rows: output rows; rw: windows a row sums).  The
+// widest lag block that still gives kPtFill workgroups with one window a unit (the
+// tile beyond the block's bands costs 1 in 4 TPW), then as many units a row as fill
+// the chip that often: a row's windows in G runs, or each window's samples in ns
+// parts of at least 512.  One workgroup a lag block ran 2.7 ms for 3 stations x 14
+// windows of 2879 samples (42 workgroups), the split 0.25 ms.
+constexpr long long kPtFill = 3072;
+
+int pt_tpw(long long rows, int rw, int L)
+{
+    return rows * rw * ((L + 32 * pt_bands(4) - 1) / (32 * pt_bands(4))) >= kPtFill / 2 ? 4 : 2;
+}
+
+PtSplit pt_split(long long rows, int rw, int N, int L, int tpw)
+{
+    PtSplit s{1, 1, (L + 32 * pt_bands(tpw) - 1) / (32 * pt_bands(tpw))};
+    const long long want = (kPtFill + rows * s.nblk - 1) / (rows * s.nblk);
+    if (want <= rw) {
+        s.G = (int)want;
+    } else {
+        s.ns = (int)std::min<long long>((want + rw - 1) / rw, std::max(1, N / 512));
+        s.G = rw * s.ns;
+    }
+    return s;
+}
+
+template <int TPW>
+int launch_pt(int fn, const cf32 *d_phi, int S, int W, int N, int lag_first, int L, float V, double div, int mode,
+              const PtSplit &sp, long long blocks, float *d_y, int out_ld, int out_off, double *part, hipStream_t st)
+{
+    const dim3 g((unsigned)blocks), b(64 * kPtWaves);
+#define FPCC_PT(FN)                                                                                               \
+    hipLaunchKernelGGL((k_pcc_time<FN, TPW>), g, b, 0, st, d_phi, S, W, N, lag_first, L, V, div, mode, sp, d_y, out_ld, \
+                       out_off, part)
+    switch (fn) {
+    case PT_SQRT: FPCC_PT(PT_SQRT); break;
+    case PT_SQUARE: FPCC_PT(PT_SQUARE); break;
+    case PT_HWPOW: FPCC_PT(PT_HWPOW); break;
+    default: FPCC_PT(PT_POW); break;
+    }
+#undef FPCC_PT
+    FPCC_CHECK(hipGetLastError());
+    return 0;
+}
+
+}  // namespace
+
+size_t pcc_time_scratch(int S, int W, int N, int L, int mode)
+{
+    if (L <= 0) return 0;
+    const long long P = (long long)S * (S - 1) / 2, rows = mode == 0 ? P * W : P;
+    const int rw = mode == 0 ? 1 : W;
+    const PtSplit sp = pt_split(rows, rw, N, L, pt_tpw(rows, rw, L));
+    return sp.G > 1 ? sizeof(double) * (size_t)rows * sp.G * (size_t)L : 0;
 }
 
 int launch_pcc_time(const cf32 *d_phi, int S, int W, int N, int lag_first, int L, double v, int pcc1, int mode,
-                    float *d_y, int out_ld, int out_off, hipStream_t st)
+                    float *d_y, int out_ld, int out_off, double *part, hipStream_t st)
 {
     if (L <= 0) return 0;
-    const int P = S * (S - 1) / 2;
-    dim3 grid((L + kPtLags - 1) / kPtLags, mode == 0 ? P * W : P);
+    const long long P = (long long)S * (S - 1) / 2, rows = mode == 0 ? P * W : P;
+    if (!rows) return 0;
+    const int rw = mode == 0 ? 1 : W;
+    const int tpw = pt_tpw(rows, rw, L);
+    PtSplit sp = pt_split(rows, rw, N, L, tpw);
+    if (!part) sp.G = sp.ns = 1;
+    const long long blocks = rows * sp.G * sp.nblk;
+    if (blocks > 0x7fffffff) {
+        fprintf(stderr, "fastpcc: %lld lag blocks exceed one launch\n", blocks);
+        return -1;
+    }
     const float V = (float)(v / 2);
-    const double div_pow = pow(2.0, (double)V);
+    // PCC1, and PCC-v at v = 1 (|.|^2 to the power 1/2), take square roots; PCC-v at
+    // v = 2 takes the squared magnitudes themselves (powf(x, 1) = x)
+    const int fn = pcc1 || V == 0.5f ? PT_SQRT : V == 1.0f ? PT_SQUARE : V > 0.f ? PT_HWPOW : PT_POW;
+    // per lag: sum / (2 count) (:276) or sum / (2^(v/2) count) (:334), over the windows of a row
+    const double div = (pcc1 ? 2.0 : pow(2.0, (double)V)) * rw;
     ProfScope prof(pcc1 ? "pcc1_time" : "pccv_time", st);
-    hipLaunchKernelGGL(k_pcc_time, grid, dim3(kPtLags), 0, st, d_phi, S, W, N, lag_first, L, pcc1, V, div_pow, mode,
-                       d_y, out_ld, out_off);
+    int r;
+    if (tpw == 4) r = launch_pt<4>(fn, d_phi, S, W, N, lag_first, L, V, div, mode, sp, blocks, d_y, out_ld, out_off, part, st);
+    else r = launch_pt<2>(fn, d_phi, S, W, N, lag_first, L, V, div, mode, sp, blocks, d_y, out_ld, out_off, part, st);
+    if (r || sp.G == 1) return r;
+    hipLaunchKernelGGL(k_pcc_time_sum, dim3((L + 255) / 256, (unsigned)rows), dim3(256), 0, st, part, N, lag_first, L,
+                       sp.G, div, d_y, out_ld, out_off);
     FPCC_CHECK(hipGetLastError());
     return 0;
 }

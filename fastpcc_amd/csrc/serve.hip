@@ -73,7 +73,7 @@ struct Request {
     fpcc_job dev_job{};  // compact device layout: station_stride = W*N
     const float *x = nullptr;
     float *y = nullptr;
-    size_t x_bytes = 0, y_bytes = 0, ws_bytes = 0;
+    size_t x_bytes = 0, y_bytes = 0, ws_bytes = 0, ws_need = 0;
     bool x_pinned = false, y_pinned = false;
     size_t off_x = 0, off_y = 0, off_ws = 0, off_sx = 0, off_sy = 0;  // arena offsets
     int state = FPCC_REQ_QUEUED, rc = 0;
@@ -496,7 +496,7 @@ int reserve_cached(Server *s, Request &r)
         r.sub_job = r.dev_job;
         r.sub_job.n_stations = std::max(2, M);
         r.xs_bytes = r.sub_job.n_stations * row;
-        r.wss_bytes = fpcc_workspace_size(&r.sub_job);
+        r.wss_bytes = job_workspace_need(&r.sub_job);  // its station stage alone
         size_t so[kMaxRegions], sp[kMaxRegions];
         if (!r.wss_bytes || job_station_regions(&r.sub_job, so, sp) != r.nreg) return -1;
         for (int k = 0; k < r.nreg; ++k) r.sub_off[k] = so[k];
@@ -889,6 +889,7 @@ int make_request(Server *s, const fpcc_request *req, std::shared_ptr<Request> &o
     r->x_bytes = (size_t)j.n_stations * r->dev_job.station_stride * sizeof(float);
     r->y_bytes = ylen * sizeof(float);
     r->ws_bytes = fpcc_workspace_size(&r->dev_job);
+    r->ws_need = fpcc::job_workspace_need(&r->dev_job);
     const size_t last = (size_t)(j.n_stations - 1) * j.station_stride + (size_t)j.n_windows * j.win_len - 1;
     r->x_pinned = fpcc::is_pinned(req->x) && fpcc::is_pinned(req->x + last);
     r->y_pinned = fpcc::is_pinned(req->y) && fpcc::is_pinned(req->y + ylen - 1);
@@ -910,7 +911,9 @@ int make_request(Server *s, const fpcc_request *req, std::shared_ptr<Request> &o
 
 int enqueue(Server *s, std::shared_ptr<Request> &r, unsigned long long *id)
 {
-    const size_t dfoot = Arena::round(r->x_bytes) + Arena::round(r->y_bytes) + Arena::round(r->ws_bytes);
+    const size_t io = Arena::round(r->x_bytes) + Arena::round(r->y_bytes);
+    if (io + Arena::round(r->ws_bytes) > s->darena.size()) r->ws_bytes = r->ws_need;  // without its optional scratch
+    const size_t dfoot = io + Arena::round(r->ws_bytes);
     const size_t hfoot = (r->x_pinned ? 0 : Arena::round(r->x_bytes)) + (r->y_pinned ? 0 : Arena::round(r->y_bytes));
     if (s->stop) return -1;
     if (dfoot > s->darena.size() || hfoot > s->harena.size()) {

@@ -162,7 +162,9 @@ typedef struct {
 
 /* Number of output floats for a job (0 if the job is invalid). */
 size_t fpcc_output_len(const fpcc_job *job);
-/* Device workspace bytes fpcc_allpairs_device needs for a job. */
+/* Device workspace bytes for a job (PCC1 and PCC-v of few pairs include a scratch of
+ * at most some MB that spreads their sums over the chip; they also run without it,
+ * more slowly, in the n_stations * n_windows * win_len phasors of 8 bytes alone). */
 size_t fpcc_workspace_size(const fpcc_job *job);
 /* Device buffers, stream-ordered on `stream` (a hipStream_t, NULL = default
  * stream); no allocation, no synchronisation.  Returns 0 or an error code. */

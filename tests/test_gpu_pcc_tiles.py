@@ -1,0 +1,96 @@
+"""Time-domain PCC1 / PCC-v where the tiled kernel can go wrong: lag blocks of 224 and
+480 lags (bands of 32), chunks of 512 samples, split and unsplit launches, and the
+records that decide between its two ways of summing PCC1's terms."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from fastpcc_amd import _lib, api
+
+pytestmark = pytest.mark.gpu
+# A term is in [-2, 2]; its half-angle phasors are rounded to 2^-25 of each component,
+# products of them are exact in three bf16 parts and summed in FP32 (a few 2^-23 of a
+# term), a dropped correction is at most 2^-24, and the FP32 analytic signal moves a
+# phasor by about 3e-7 / |z|, which averages out: 1e-6 over 400 terms and more.  Short
+# overlaps can hold single phasors of small |z| (1e-5, as the other tests).
+TOL, TOL_SHORT, LONG = 1e-6, 1e-5, 400
+
+
+def _records(S, W, N, seed, what):
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal((S, W, N)).astype(np.float32)
+    n = np.arange(N)
+    if what == "event":  # a decaying event far above the noise: large regulariser differences
+        x[:, 0] += (300 * np.exp(-n / 40.0) * np.sin(0.7 * n)).astype(np.float32)
+    elif what == "silent":
+        x[1, -1] = 0
+        x[0, 0, : N // 2] = 0
+    elif what == "antiphase":  # one modulated tone and its negative: |a+b| = |d| at every sample
+        tone = ((1.5 + np.sin(2 * np.pi * 3 * n / N)) * np.sin(0.9 * n)).astype(np.float32)
+        x[0] = tone
+        x[1:] = -tone
+    return x.reshape(S, W * N)
+
+
+def _check(y, yr, N, lag1, lag2, tol=TOL):
+    long_ = N - np.abs(np.arange(lag1, lag2 + 1)) >= LONG
+    d = np.abs(y - yr)
+    err = [float(d[..., m].max()) if m.any() else 0.0 for m in (long_, ~long_)]
+    print(f"  max|gpu-fp64| {err[0]:.2e} (overlap >= {LONG}), {err[1]:.2e}")
+    assert err[0] <= tol and err[1] <= TOL_SHORT
+
+
+@pytest.mark.parametrize("S,W,N,lag1,lag2,stack", [
+    (2, 1, 511, 0, 0, "none"), (2, 1, 512, -16, 15, "none"), (2, 1, 513, -16, 16, "none"),
+    (3, 2, 1025, -112, 111, "none"), (3, 2, 1024, -112, 112, "plain"), (2, 5, 1600, -240, 239, "plain"),
+    (2, 1, 5003, -240, 240, "none"), (40, 24, 64, -31, 31, "none"), (40, 24, 64, -63, 63, "plain"),
+    (24, 8, 700, 37, 690, "plain"), (2, 1, 2, -1, 1, "none")])
+@pytest.mark.parametrize("kind,v", [("pcc1", 1.0), ("pccv", 2.0), ("pccv", 1.5)])
+def test_tile_edges(fp, orc, S, W, N, lag1, lag2, stack, kind, v):
+    if N == 2 and kind == "pccv":
+        pytest.skip("one length of this kind is enough")
+    x = _records(S, W, N, S * N + W, "noise")
+    y = fp.allpairs(x, W, N, lag1, lag2, kind=kind, stack=stack, v=v)
+    yr = orc.allpairs(kind, x, W, N, lag1, lag2, stacked=stack != "none", f64=True, v=v)
+    _check(y, yr, N, lag1, lag2)
+
+
+@pytest.mark.parametrize("what", ["event", "silent", "antiphase"])
+@pytest.mark.parametrize("kind,v", [("pcc1", 1.0), ("pccv", 1.5)])
+def test_records_on_both_ways(fp, orc, what, kind, v):
+    S, W, N = 4, 3, 1800
+    x = _records(S, W, N, 7, what)
+    y = fp.allpairs(x, W, N, -300, 300, kind=kind, stack="none", v=v)
+    yr = orc.allpairs(kind, x, W, N, -300, 300, stacked=False, f64=True, v=v)
+    # the FP32 transform's error is 3e-7 of the window's rms: half of a silent record holds
+    # the Hilbert transform's tail of the other half, |z| about 0.05 of the rms, and the
+    # event's window is noise of 0.05 of the rms too, so its phasors are off by 6e-6
+    _check(y, yr, N, -300, 300, tol=TOL if what == "antiphase" else TOL_SHORT)
+
+
+@pytest.mark.parametrize("stack", ["none", "plain"])
+def test_workspace_without_the_split_scratch(fp, hip, stack):
+    """A workspace that holds the phasors alone runs unsplit; sums in another order."""
+    S, W, N = 3, 4, 1500
+    x = _records(S, W, N, 3, "noise")
+    job = api.make_job("pcc1", S, W, N, -200, 200, stack)
+    lib, jp = _lib.lib(), ctypes.byref(job)
+    total, need = lib.fpcc_workspace_size(jp), -(-S * W * N * 8 // 256) * 256
+    assert total > need
+    nout = lib.fpcc_output_len(jp)
+    dx, dy, ws = hip.alloc(x.nbytes), hip.alloc(4 * nout), hip.alloc(total)
+    hip.h2d(dx, x)
+
+    def run(size):
+        y = np.full(nout, np.nan, dtype=np.float32)
+        hip.h2d(dy, y)
+        r = lib.fpcc_allpairs_device(jp, ctypes.c_void_p(dx), ctypes.c_void_p(dy), ctypes.c_void_p(ws), size, None)
+        hip.d2h(y, dy)
+        return r, y
+
+    (r0, full), (r1, small) = run(total), run(need)
+    assert r0 == 0 and r1 == 0
+    # FP64 sums of the same FP32 partial sums of at most 64 terms, cut at other samples
+    assert np.abs(small - full).max() <= 2e-8
+    assert run(need - 256)[0] == -1
