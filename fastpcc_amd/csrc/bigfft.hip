@@ -6,7 +6,8 @@
 #include <string>
 #include "../../include/fastpcc.h"
 #include "bigfft.hpp"
-#include "edge.hpp"
+#include "tile_fft.hpp"
+#include "lagwin.hpp"
 #include "kernels.hpp"
 #include "profile.hpp"
 #include "pairs.hpp"
@@ -106,13 +107,10 @@ const BigPlan &big_plan(int n)
     return cache.emplace(std::make_pair(dev, n), make_big_plan(n)).first->second;
 }
 
-// index of W_n^{c r} in the full table: c < N2 and r < N1, so c*r < n
-// W_n^{c r} from the two-factor table of get_split_twiddles (c r < n): two small
-// cached lookups instead of a gather over an n-entry table
+// W_n^{c r}, c r < n
 __device__ __forceinline__ cf32 tw_cr(const cf32 *__restrict__ twN, int c, int r)
 {
-    const unsigned m = (unsigned)c * (unsigned)r;
-    return cmul(twN[kTwLo + m / kTwLo], twN[m % kTwLo]);
+    return tw_m(twN, (unsigned)c * (unsigned)r);
 }
 
 // Job-table launch (BATCH): batch index b runs over the rows of several jobs; job j
@@ -126,95 +124,7 @@ __device__ __forceinline__ int batch_job(const RealBatch &jb, int b)
     return j;
 }
 
-// Compile-time batched transforms for the common splits (2^17 .. 2^19 as 256 x
-// 512 .. 256 x 2048): NTR transforms of NPT points transform in place in one LDS
-// buffer, transform t at t * LDT, point i at ct_pad(i) (one pad slot per 16
-// values), 256 threads, each pass reading all of a thread's butterflies before
-// writing.  Columns: 16 x 256 points, radix 16 x 16, stride 274; rows: 4 x 512
-// (8 x 8 x 8, stride 544) or 4 x 1024 (16 x 8 x 8, stride 1088).  The strides keep
-// the loads, passes and stores within 1.5x of conflict-free LDS access.
 constexpr int kCtN1 = 256, kCtLD = 274;
-
-template <int NPT, int NTR, int LDT, int DIR, int R, int NS>
-__device__ __forceinline__ void ctb_pass(cf32 *lds, const cf32 *__restrict__ tw)
-{
-    constexpr int NBF = NPT / R, TOT = NTR * NBF, BPT = (TOT + 255) / 256;
-    cf32 v[BPT][R];
-#pragma unroll
-    for (int i = 0; i < BPT; ++i) {
-        const int bb = threadIdx.x + 256 * i;
-        if (TOT % 256 == 0 || bb < TOT) {
-            const int t = bb / NBF, b = bb % NBF;
-#pragma unroll
-            for (int r = 0; r < R; ++r) v[i][r] = lds[t * LDT + ct_pad(b + r * NBF)];
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < BPT; ++i) {
-        const int bb = threadIdx.x + 256 * i;
-        if (TOT % 256 == 0 || bb < TOT) {
-            const int t = bb / NBF, b = bb % NBF;
-            const int k = b % NS;
-            if (NS > 1) {
-#pragma unroll
-                for (int r = 1; r < R; ++r) {
-                    cf32 w = tw[(r - 1) * NS + k];
-                    if (DIR > 0) w.y = -w.y;
-                    v[i][r] = cmul(v[i][r], w);
-                }
-            }
-            Dft<R, DIR>::run(v[i]);
-            const int base = (b - k) * R + k;
-#pragma unroll
-            for (int r = 0; r < R; ++r) lds[t * LDT + ct_pad(base + r * NS)] = v[i][r];
-        }
-    }
-    __syncthreads();
-}
-
-// Register-ended passes of a tile's in-place transforms (transform t's point p at
-// lds[t * LDT + ct_pad(p)]), one butterfly b of transform t a call.  First pass
-// (stride 1): the butterfly's inputs, points b + r NPT/R, are in v; its outputs go
-// to LDS (the caller puts a barrier after every thread's call).
-template <int NPT, int LDT, int DIR, int R>
-__device__ __forceinline__ void ctb_first_regs(cf32 *v, int t, int b, cf32 *lds)
-{
-    Dft<R, DIR>::run(v);
-#pragma unroll
-    for (int r = 0; r < R; ++r) lds[t * LDT + ct_pad(b * R + r)] = v[r];
-}
-// Last pass (stride NPT/R): the butterfly's outputs, points b + r NPT/R, stay in v.
-template <int NPT, int LDT, int DIR, int R>
-__device__ __forceinline__ void ctb_last_regs(const cf32 *lds, int t, int b, cf32 *v, const cf32 *__restrict__ tw)
-{
-    constexpr int NS = NPT / R;
-#pragma unroll
-    for (int r = 0; r < R; ++r) v[r] = lds[t * LDT + ct_pad(b + r * NS)];
-#pragma unroll
-    for (int r = 1; r < R; ++r) {
-        cf32 w = tw[(r - 1) * NS + b];
-        if (DIR > 0) w.y = -w.y;
-        v[r] = cmul(v[r], w);
-    }
-    Dft<R, DIR>::run(v);
-}
-
-template <int NPT, int NTR, int LDT, int DIR, int NS, int OFF, int R, int... Rest>
-__device__ __forceinline__ void ctb_passes(cf32 *lds, const cf32 *__restrict__ tw)
-{
-    ctb_pass<NPT, NTR, LDT, DIR, R, NS>(lds, tw + OFF);
-    if constexpr (sizeof...(Rest) > 0) ctb_passes<NPT, NTR, LDT, DIR, NS * R, OFF + (R - 1) * NS, Rest...>(lds, tw);
-}
-
-// tw: the per-pass twiddles of the plan with radices Rs (in that order)
-template <int NPT, int NTR, int LDT, int DIR, int... Rs>
-__device__ __forceinline__ cf32 *ctb_fft(cf32 *lds, const cf32 *__restrict__ tw)
-{
-    static_assert((Rs * ... * 1) == NPT, "radices must multiply to NPT");
-    ctb_passes<NPT, NTR, LDT, DIR, 1, 0, Rs...>(lds, tw);
-    return lds;
-}
 
 template <int DIR>
 __device__ __forceinline__ cf32 *ct_cols_fft(cf32 *lds, const cf32 *__restrict__ tw)
@@ -336,33 +246,7 @@ k_big_cols(ColArgs a, int N1, int N2, FftPlan p1, const cf32 *__restrict__ tw1, 
             long long d = g - a.lag0;  // in (-n, 2n): lag0 is in (-n, n)
             if (d < 0) d += n;
             if (d >= n) d -= n;
-            const int l = (int)d;
-            if (l < a.L) {
-                const int lag = a.lag0 + l;
-                double o = (double)(a.scale * v.x);
-                const int m = a.Nsig - abs(lag);
-                if (a.edge && m > 0 && m < a.K) {
-                    // short overlap: the FP32 transform's absolute error, divided by
-                    // the overlap's small energy, would dominate; sum it exactly
-                    int ei = i, ej = j;
-                    if (a.norm != 1) pair_index(p, a.S, ei, ej);
-                    const int w0 = a.esum ? 0 : w, w1 = a.esum ? a.Wall : w + 1;
-                    const double c = edge_corr(a.edge, a.K, a.Wall, ei, ej, w0, w1, lag, m, a.norm == 2);
-                    o = c * (double)a.scale * (double)n;  // the transform's scale: v.x is n c
-                }
-                if (a.norm == 1) {
-                    const double *P1 = a.E + (long long)(i * a.Wfull + w) * a.lde;
-                    const double *P2 = a.E + (long long)(j * a.Wfull + w) * a.lde;
-                    const int N = a.Nsig;
-                    const int a1 = max(0, -lag), b1 = min(N, N - lag);
-                    const int a2 = max(0, lag), b2 = min(N, N + lag);
-                    o = o / sqrt((P1[b1] - P1[a1]) * (P2[b2] - P2[a2]));
-                } else if (a.norm == 2) {
-                    o = o / (double)(a.Nsig - abs(lag));
-                }
-                if (a.accumulate) a.y[(long long)p * a.L + l] += (float)o;
-                else a.y[((long long)p * a.Wfull + w) * a.L + l] = (float)o;
-            }
+            if (d < a.L) lagwin_store(a, p, w, i, j, n, (int)d, v.x);
         }
     };
     bool regs = false;  // transformed in registers and emitted

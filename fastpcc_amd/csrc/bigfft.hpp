@@ -111,6 +111,13 @@ int bluestein_n(int N);
 int bluestein_tables(int N, int n, cf32 *chirp, cf32 *T, hipStream_t st);
 
 struct RealBatch;
+// Pair stage without the passes through HBM (longpair.hip): the spectra (or folded
+// rows) of ra (ROW_INV_CROSS or ROW_INV_PLAIN) to the lags of ca (COL_INV_LAGWIN), the
+// partial sums in the rows of ra.dst; real: spectra of real signals.  false if the
+// split or the lag window does not qualify.
+bool long_pair_ok(const BigPlan &bp, int lag0, int L);
+int run_long_pair(const BigPlan &bp, const RowArgs &ra, const ColArgs &ca, bool real, int nbatch, hipStream_t st,
+                  const char *name);
 int run_cols(const BigPlan &bp, const ColArgs &a, int nbatch, hipStream_t st, const char *name);
 // COL_FWD_INPUT / ROW_FWD_PLAIN over the station-windows of several jobs (x, stride,
 // W, N and destination rows from the job table; the other fields from a).

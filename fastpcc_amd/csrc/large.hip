@@ -403,7 +403,6 @@ int large_pair_stage(int kind, int stack, int S, int W, int N, int Nz, int lag0,
             const int np = std::min(65535, P - p0);
             ra.src = G + (long long)p0 * ldg;
             ra.dst = G + (long long)p0 * ldg;
-            if ((r = run_rows(bz, ra, np, st, "pair_inv_rows"))) return r;
             ColArgs ca;
             ca.op = COL_INV_LAGWIN;
             ca.src = G + (long long)p0 * ldg;
@@ -422,6 +421,11 @@ int large_pair_stage(int kind, int stack, int S, int W, int N, int Nz, int lag0,
                 ca.Wall = W;
                 ca.esum = 1;
             }
+            if (long_pair_ok(bz, lag0, L)) {
+                if ((r = run_long_pair(bz, ra, ca, false, np, st, "pair_long"))) return r;
+                continue;
+            }
+            if ((r = run_rows(bz, ra, np, st, "pair_inv_rows"))) return r;
             if ((r = run_cols(bz, ca, np, st, "pair_inv_cols"))) return r;
         }
         return 0;
@@ -478,6 +482,10 @@ int large_pair_stage(int kind, int stack, int S, int W, int N, int Nz, int lag0,
             ra.pair0 = pair0;
             ca.pair0 = pair0;
             ca.y = y;
+            if (long_pair_ok(bz, lag0, L)) {
+                if ((r = run_long_pair(bz, ra, ca, kind != FPCC_PCC2, nbt, st, "pair_long"))) return r;
+                continue;
+            }
             if ((r = run_rows(bz, ra, nbt, st, "pair_cross_rows"))) return r;
             if ((r = run_cols(bz, ca, nbt, st, "pair_inv_cols"))) return r;
         }

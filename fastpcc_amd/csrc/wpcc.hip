@@ -308,7 +308,6 @@ int wpcc_pair_stage(int S, int W, int N, const WFamily &f, int lag0, int L, bool
         ra.dst = G;
         ra.bstride = ldg;
         ra.S = 1;
-        if ((r = run_rows(bp, ra, P, st, "wpcc_pair_inv_rows"))) return r;
         ColArgs ca{};
         ca.op = COL_INV_LAGWIN;
         ca.src = G;
@@ -321,6 +320,11 @@ int wpcc_pair_stage(int S, int W, int N, const WFamily &f, int lag0, int L, bool
         ca.wsel = per_window ? w : 0;
         ca.Wfull = per_window ? W : 1;
         ca.scale = (float)(per_window ? C : C / W);
+        if (long_pair_ok(bp, lag0, L)) {
+            if ((r = run_long_pair(bp, ra, ca, false, P, st, "wpcc_pair_long"))) return r;
+            continue;
+        }
+        if ((r = run_rows(bp, ra, P, st, "wpcc_pair_inv_rows"))) return r;
         if ((r = run_cols(bp, ca, P, st, "wpcc_pair_inv_cols"))) return r;
     }
     return 0;
