@@ -114,8 +114,9 @@ struct RealBatch;
 // Pair stage without the passes through HBM (longpair.hip): the spectra (or folded
 // rows) of ra (ROW_INV_CROSS or ROW_INV_PLAIN) to the lags of ca (COL_INV_LAGWIN), the
 // partial sums in the rows of ra.dst; real: spectra of real signals.  false if the
-// split or the lag window does not qualify.
-bool long_pair_ok(const BigPlan &bp, int lag0, int L);
+// split, the lag window or the number of items (each the sum of wsum windows) does not
+// qualify.
+bool long_pair_ok(const BigPlan &bp, int lag0, int L, long long nbatch, int wsum);
 int run_long_pair(const BigPlan &bp, const RowArgs &ra, const ColArgs &ca, bool real, int nbatch, hipStream_t st,
                   const char *name);
 int run_cols(const BigPlan &bp, const ColArgs &a, int nbatch, hipStream_t st, const char *name);

@@ -9,6 +9,10 @@ namespace fpcc {
 // PCC2 station stage: F[s*W+w][Nz] = FFT_Nz(pad(AmpNormf(analytic_N(x_sw))))
 int launch_station_pcc(const float *d_x, long long station_stride, int S, int W, int N, int Nz, cf32 *d_F,
                        hipStream_t st);
+// Analytic signals of S*W windows in LDS (analytic.hip) into rows Z of N values, their
+// max|z|^2 into mx; even N whose half is 7-smooth and fits (analytic_lds_ok).
+bool analytic_lds_ok(int N);
+int launch_analytic_lds(const float *x, long long stride, int S, int W, int N, cf32 *Z, float *mx, hipStream_t st);
 // Half-angle phasors (pcc_time.hip) in place of `rows` rows of N analytic samples.
 int launch_half_phasor_rows(cf32 *d_z, int rows, int N, hipStream_t st);
 // Half-angle phasors only (analytic signal + AmpNormf, pcc_time.hip), phi[s*W+w][N].

@@ -234,6 +234,7 @@ static int analytic_bluestein(const float *x, long long stride, int S, int W, in
 static int analytic_big(const float *x, long long stride, int S, int W, int N, cf32 *Z, float *mx, cf32 *B,
                         hipStream_t st)
 {
+    if (analytic_lds_ok(N)) return launch_analytic_lds(x, stride, S, W, N, Z, mx, st);
     const BigPlan &bp = big_plan(N);
     if (!bp.ok) return analytic_bluestein(x, stride, S, W, N, Z, mx, B, st);
     const int SW = S * W;
@@ -421,7 +422,7 @@ int large_pair_stage(int kind, int stack, int S, int W, int N, int Nz, int lag0,
                 ca.Wall = W;
                 ca.esum = 1;
             }
-            if (long_pair_ok(bz, lag0, L)) {
+            if (long_pair_ok(bz, lag0, L, np, 1)) {
                 if ((r = run_long_pair(bz, ra, ca, false, np, st, "pair_long"))) return r;
                 continue;
             }
@@ -482,7 +483,7 @@ int large_pair_stage(int kind, int stack, int S, int W, int N, int Nz, int lag0,
             ra.pair0 = pair0;
             ca.pair0 = pair0;
             ca.y = y;
-            if (long_pair_ok(bz, lag0, L)) {
+            if (long_pair_ok(bz, lag0, L, nbt, wsum ? W : 1)) {
                 if ((r = run_long_pair(bz, ra, ca, kind != FPCC_PCC2, nbt, st, "pair_long"))) return r;
                 continue;
             }

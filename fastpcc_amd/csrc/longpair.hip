@@ -252,11 +252,16 @@ int launch_lp(const LongArgs &a, int src, int blocks, hipStream_t st)
 // Rows of 512, 1024 or 2048 bins (the splits of 2^14 .. 2^20), at least one whole unit,
 // lags whose sums stay in registers (|n1| H <= 3072: within +-6144; the sums cost 2 |n1|
 // multiply-adds a bin) and fit the rows a share read.
-bool long_pair_ok(const BigPlan &bp, int lag0, int L)
+// And work for half the chip: the units of all items are its workgroups, against one
+// for every four rows of the two passes.  1-bit, one window: 72 units 0.98x of the two
+// passes' speed, 144 1.09x, 182 1.22x (N 10000, 24000, 10000); with windows summed
+// unit by unit 6 units ran at half their speed (3 pairs x 40 windows of 12001).
+bool long_pair_ok(const BigPlan &bp, int lag0, int L, long long nbatch, int wsum)
 {
     if (!bp.ok || (bp.n2 != 512 && bp.n2 != 1024 && bp.n2 != 2048)) return false;
     const int H = bp.n2 / 2, PU = 2048 / H, U = bp.n1 / (2 * PU);
     if (U < 1 || (bp.n1 & (bp.n1 - 1))) return false;
+    if (nbatch * U < (wsum > 1 ? 512 : 128)) return false;
     const int A = lp_reach(lag0, L, H);
     return A * H <= 3072 && (long long)(2 * A + 1) * H <= (long long)U * 4096;
 }
@@ -265,7 +270,7 @@ int run_long_pair(const BigPlan &bp, const RowArgs &ra, const ColArgs &ca, bool 
                   const char *name)
 {
     if (nbatch <= 0) return 0;
-    if (!long_pair_ok(bp, ca.lag0, ca.L) || nbatch > 65535) return -1;
+    if (!long_pair_ok(bp, ca.lag0, ca.L, nbatch, ra.wsum ? ra.Wfull : 1) || nbatch > 65535) return -1;
     const int H = bp.n2 / 2, PU = 2048 / H, U = bp.n1 / (2 * PU);
     LongArgs a{};
     const bool gram = ra.op == ROW_INV_PLAIN;

@@ -320,7 +320,7 @@ int wpcc_pair_stage(int S, int W, int N, const WFamily &f, int lag0, int L, bool
         ca.wsel = per_window ? w : 0;
         ca.Wfull = per_window ? W : 1;
         ca.scale = (float)(per_window ? C : C / W);
-        if (long_pair_ok(bp, lag0, L)) {
+        if (long_pair_ok(bp, lag0, L, P, 1)) {
             if ((r = run_long_pair(bp, ra, ca, false, P, st, "wpcc_pair_long"))) return r;
             continue;
         }
