@@ -124,12 +124,25 @@ __device__ __forceinline__ int batch_job(const RealBatch &jb, int b)
     return j;
 }
 
-constexpr int kCtN1 = 256, kCtLD = 274;
+// Columns of 32 .. 256 points (the splits of 2^14 .. 2^19): 16 columns a workgroup, a
+// first-radix butterfly a thread (8 x 4, 8 x 8, 16 x 8, 16 x 16).  The runtime plan ran the
+// zero-padded 32768-point columns (N1 64) of 1298 windows in 324 us, this 165 us, bound by
+// HBM and the AmpNormf square roots.  Columns of 32 and 64 points with the lag epilogue
+// keep the runtime plan: several points a thread lengthen the epilogues of the few
+// items that come here (GNCC, 3 pairs: 0.78x and 0.90x of its speed); tiles of 4096
+// points (64 columns of 64) left single transforms too few workgroups (0.94x).
+// LDS stride of a column (one pad slot per 16; odd for short columns, whose lanes run
+// across columns): 0 if not specialised.
+__host__ __device__ constexpr int ct_col_ld(int n1) { return n1 == 256 ? 274 : n1 == 128 || n1 == 64 || n1 == 32 ? n1 + n1 / 16 + 1 : 0; }
+__host__ __device__ constexpr int ct_col_r1(int n1) { return n1 <= 64 ? 8 : 16; }  // first radix, points a thread
+__host__ __device__ constexpr int ct_col_threads(int n1) { return n1 ? kBigCols * n1 / ct_col_r1(n1) : 256; }
 
-template <int DIR>
+template <int CTN1, int DIR>
 __device__ __forceinline__ cf32 *ct_cols_fft(cf32 *lds, const cf32 *__restrict__ tw)
 {
-    return ctb_fft<kCtN1, kBigCols, kCtLD, DIR, 16, 16>(lds, tw);
+    ctb_passes<ct_col_threads(CTN1), CTN1, kBigCols, ct_col_ld(CTN1), DIR, 1, 0, ct_col_r1(CTN1),
+               CTN1 / ct_col_r1(CTN1)>(lds, tw);
+    return lds;
 }
 
 // rows: stride of the in-place layout for N2 (0: not specialised)
@@ -142,19 +155,22 @@ __device__ __forceinline__ cf32 *ct_rows_fft(cf32 *lds, const cf32 *__restrict__
     else return ctb_fft<1024, kBigRows, ct_row_ld(1024), DIR, 16, 8, 8>(lds, tw);
 }
 
-template <bool BATCH, bool CT>
-__global__ void __launch_bounds__(256)
+// CTN1: compile-time column length (0: the runtime plan)
+template <bool BATCH, int CTN1>
+__global__ void __launch_bounds__(ct_col_threads(CTN1))
 k_big_cols(ColArgs a, int N1, int N2, FftPlan p1, const cf32 *__restrict__ tw1, const cf32 *__restrict__ twN,
            RealBatch jb)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     // column t, point r at cix(t, r): padded column stride N1 + 1 with ping-pong
-    // buffers, or the in-place layout of ct_cols_fft (N1 = 256, tw1 its twiddles)
-    const int ld = CT ? kCtLD : N1 + 1;
-    auto cix = [&](int t, int r) { return CT ? t * kCtLD + ct_pad(r) : t * ld + r; };
+    // buffers, or the in-place layout of ct_cols_fft (tw1 its twiddles)
+    constexpr bool CT = CTN1 != 0;
+    constexpr int NC = kBigCols, LDC = ct_col_ld(CTN1), NT = ct_col_threads(CTN1);
+    const int ld = CT ? LDC : N1 + 1;
+    auto cix = [&](int t, int r) { return CT ? t * LDC + ct_pad(r) : t * ld + r; };
     cf32 *buf0 = reinterpret_cast<cf32 *>(smem_raw);
-    cf32 *buf1 = buf0 + kBigCols * ld;
-    float *red = reinterpret_cast<float *>(CT ? buf1 : buf1 + kBigCols * ld);
+    cf32 *buf1 = buf0 + NC * ld;
+    float *red = reinterpret_cast<float *>(CT ? buf1 : buf1 + NC * ld);
     int b = blockIdx.y;
     if (BATCH) {
         const int j = batch_job(jb, b);
@@ -176,7 +192,7 @@ k_big_cols(ColArgs a, int N1, int N2, FftPlan p1, const cf32 *__restrict__ tw1, 
             a.maxbuf = jb.mx[j];
         }
     }
-    const int c0 = blockIdx.x * kBigCols;
+    const int c0 = blockIdx.x * NC;
     const long long base = (long long)b * a.bstride;
     const long long sbase = (long long)b * (a.src_bstride ? a.src_bstride : a.bstride);
     const int n = N1 * N2;
@@ -251,16 +267,16 @@ k_big_cols(ColArgs a, int N1, int N2, FftPlan p1, const cf32 *__restrict__ tw1, 
     };
     bool regs = false;  // transformed in registers and emitted
     if constexpr (CT) {
-        // all of a thread's loads first (16 points of 256 columns-rows), then the work:
+        // all of a thread's loads first (8 or 16 points), then the work:
         // a loop that loads, computes and stores one point at a time waits for every load
-        constexpr int PER = kBigCols * kCtN1 / 256;
+        constexpr int PER = NC * CTN1 / NT;
         const bool xin = op == COL_FWD_INPUT || op == COL_FWD_CHIRP;
         cf32 u[PER];
         float xv[PER];
         bool in[PER];
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
-            const int idx = threadIdx.x + 256 * i, t = idx % kBigCols, r = idx / kBigCols, c = c0 + t;
+            const int idx = threadIdx.x + NT * i, t = idx % NC, r = idx / NC, c = c0 + t;
             const long long g = (long long)r * N2 + c;
             u[i] = cf32{0.f, 0.f};
             xv[i] = 0.f;
@@ -279,44 +295,52 @@ k_big_cols(ColArgs a, int N1, int N2, FftPlan p1, const cf32 *__restrict__ tw1, 
         cf32 v[PER];
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
-            const int idx = threadIdx.x + 256 * i, t = idx % kBigCols, r = idx / kBigCols, c = c0 + t;
+            const int idx = threadIdx.x + NT * i, t = idx % NC, r = idx / NC, c = c0 + t;
             v[i] = c < N2 ? start((long long)r * N2 + c, u[i], xv[i], in[i]) : cf32{0.f, 0.f};
         }
         if (op != COL_CHIRP_MID) {
-            // thread (column t, q) holds rows q + 16 i: the inputs of the first radix-16
-            // butterfly q of column t; the second pass's butterfly q gives rows q + 16 i
-            // back, the points this thread stores.  One barrier between the passes.
-            const int t = threadIdx.x % kBigCols, q = threadIdx.x / kBigCols, c = c0 + t;
-            if (inv) ctb_first_regs<kCtN1, kCtLD, +1, 16>(v, t, q, buf0);
-            else ctb_first_regs<kCtN1, kCtLD, -1, 16>(v, t, q, buf0);
+            // thread (column t, q) holds rows q + (N1/R1) i: the inputs of the first pass's
+            // butterfly q of column t.  The second pass's butterflies b (radix R2, R1/R2 a
+            // thread) give rows b + R1 r, which this thread stores (R1 = R2: its own rows).
+            // One barrier between the passes.
+            constexpr int R1 = ct_col_r1(CTN1), R2 = CTN1 / R1, NB = R1 / R2;
+            const int t = threadIdx.x % NC, q = threadIdx.x / NC;
+            if (inv) ctb_first_regs<CTN1, LDC, +1, R1>(v, t, q, buf0);
+            else ctb_first_regs<CTN1, LDC, -1, R1>(v, t, q, buf0);
             __syncthreads();
-            if (inv) ctb_last_regs<kCtN1, kCtLD, +1, 16>(buf0, t, q, v, tw1 + 15);
-            else ctb_last_regs<kCtN1, kCtLD, -1, 16>(buf0, t, q, v, tw1 + 15);
+#pragma unroll
+            for (int k = 0; k < NB; ++k) {
+                const int b2 = q + k * R2;  // (threadIdx.x + NT k) / NC: the columns stay
+                if (inv) ctb_last_regs<CTN1, LDC, +1, R2>(buf0, t, b2, v + k * R2, tw1 + (R1 - 1));
+                else ctb_last_regs<CTN1, LDC, -1, R2>(buf0, t, b2, v + k * R2, tw1 + (R1 - 1));
+            }
+            const int c = c0 + t;
+            auto row_of = [&](int i) { return q + (i / R2) * R2 + R1 * (i % R2); };
             if (fwd_out) {
                 // the step twiddles of all of a thread's points first, then the stores
                 cf32 wt[PER];
 #pragma unroll
-                for (int i = 0; i < PER; ++i) wt[i] = c < N2 ? tw_cr(twN, c, q + 16 * i) : cf32{0.f, 0.f};
+                for (int i = 0; i < PER; ++i) wt[i] = c < N2 ? tw_cr(twN, c, row_of(i)) : cf32{0.f, 0.f};
 #pragma unroll
                 for (int i = 0; i < PER; ++i)
-                    if (c < N2) a.dst[base + (long long)(q + 16 * i) * N2 + c] = cmul(v[i], wt[i]);  // W_n^{n2 k1}
+                    if (c < N2) a.dst[base + (long long)row_of(i) * N2 + c] = cmul(v[i], wt[i]);  // W_n^{n2 k1}
             } else {
 #pragma unroll
                 for (int i = 0; i < PER; ++i)
-                    if (c < N2) emit(t, q + 16 * i, v[i]);
+                    if (c < N2) emit(t, row_of(i), v[i]);
             }
             regs = true;
         } else {
 #pragma unroll
             for (int i = 0; i < PER; ++i) {
-                const int idx = threadIdx.x + 256 * i, t = idx % kBigCols, r = idx / kBigCols;
+                const int idx = threadIdx.x + NT * i, t = idx % NC, r = idx / NC;
                 buf0[cix(t, r)] = v[i];
             }
         }
     }
     if (!regs) {
-        for (int idx = threadIdx.x; !CT && idx < kBigCols * N1; idx += blockDim.x) {
-            const int t = idx % kBigCols, r = idx / kBigCols;
+        for (int idx = threadIdx.x; !CT && idx < NC * N1; idx += blockDim.x) {
+            const int t = idx % NC, r = idx / NC;
             const int c = c0 + t;
             cf32 v = cf32{0.f, 0.f};
             if (c < N2) {
@@ -350,15 +374,15 @@ k_big_cols(ColArgs a, int N1, int N2, FftPlan p1, const cf32 *__restrict__ tw1, 
         }
         __syncthreads();
         cf32 *res;
-        if (CT) res = inv ? ct_cols_fft<+1>(buf0, tw1) : ct_cols_fft<-1>(buf0, tw1);
+        if constexpr (CT) res = inv ? ct_cols_fft<CTN1, +1>(buf0, tw1) : ct_cols_fft<CTN1, -1>(buf0, tw1);
         else
-            res = inv ? fft_lds_batch<float, +1>(buf0, buf1, p1, tw1, kBigCols, ld)
-                      : fft_lds_batch<float, -1>(buf0, buf1, p1, tw1, kBigCols, ld);
+            res = inv ? fft_lds_batch<float, +1>(buf0, buf1, p1, tw1, NC, ld)
+                      : fft_lds_batch<float, -1>(buf0, buf1, p1, tw1, NC, ld);
         if (op == COL_CHIRP_MID) {
             // second transform's chirped input: conj(mask X) w = mask conj(conv) (|w| = 1)
             const int half = (a.N + 1) >> 1;
-            for (int idx = threadIdx.x; idx < kBigCols * N1; idx += blockDim.x) {
-                const int t = idx % kBigCols, r = idx / kBigCols;
+            for (int idx = threadIdx.x; idx < NC * N1; idx += blockDim.x) {
+                const int t = idx % NC, r = idx / NC;
                 const long long g = (long long)r * N2 + c0 + t;
                 float gm = 0.f;
                 if (c0 + t < N2 && g < a.N) {
@@ -370,29 +394,30 @@ k_big_cols(ColArgs a, int N1, int N2, FftPlan p1, const cf32 *__restrict__ tw1, 
                 res[cix(t, r)] = cf32{gm * v.x, -gm * v.y};
             }
             __syncthreads();
-            res = CT ? ct_cols_fft<-1>(res, tw1) : fft_lds_batch<float, -1>(res, res == buf0 ? buf1 : buf0, p1, tw1, kBigCols, ld);
+            if constexpr (CT) res = ct_cols_fft<CTN1, -1>(res, tw1);
+            else res = fft_lds_batch<float, -1>(res, res == buf0 ? buf1 : buf0, p1, tw1, NC, ld);
         }
         bool done = false;
         if constexpr (CT) {
             if (fwd_out) {
                 // the step twiddles of all of a thread's points first, then the stores
-                constexpr int PER = kBigCols * kCtN1 / 256;
+                constexpr int PER = NC * CTN1 / NT;
                 cf32 w[PER];
     #pragma unroll
                 for (int i = 0; i < PER; ++i) {
-                    const int idx = threadIdx.x + 256 * i, t = idx % kBigCols, r = idx / kBigCols, c = c0 + t;
+                    const int idx = threadIdx.x + NT * i, t = idx % NC, r = idx / NC, c = c0 + t;
                     w[i] = c < N2 ? tw_cr(twN, c, r) : cf32{0.f, 0.f};
                 }
     #pragma unroll
                 for (int i = 0; i < PER; ++i) {
-                    const int idx = threadIdx.x + 256 * i, t = idx % kBigCols, r = idx / kBigCols, c = c0 + t;
+                    const int idx = threadIdx.x + NT * i, t = idx % NC, r = idx / NC, c = c0 + t;
                     if (c < N2) a.dst[base + (long long)r * N2 + c] = cmul(res[cix(t, r)], w[i]);  // W_n^{n2 k1}
                 }
                 done = true;
             }
         }
-        for (int idx = threadIdx.x; !done && idx < kBigCols * N1; idx += blockDim.x) {
-            const int t = idx % kBigCols, r = idx / kBigCols;
+        for (int idx = threadIdx.x; !done && idx < NC * N1; idx += blockDim.x) {
+            const int t = idx % NC, r = idx / NC;
             if (c0 + t >= N2) continue;
             emit(t, r, res[cix(t, r)]);
         }
@@ -750,25 +775,41 @@ int bluestein_tables(int N, int n, cf32 *chirp, cf32 *T, hipStream_t st)
     return run_rows(bp, ra, 1, st, "bluestein_table_rows");
 }
 
+template <bool BATCH, int CTN1>
+static int launch_cols_ct(const BigPlan &bp, const ColArgs &a, const RealBatch &jb, int nbatch, hipStream_t st,
+                          const char *name)
+{
+    // compile-time in-place column transform, one LDS buffer
+    const cf32 *twc = (const cf32 *)get_order_twiddles(CTN1, {ct_col_r1(CTN1), CTN1 / ct_col_r1(CTN1)});
+    if (!twc) return -1;
+    constexpr int NC = kBigCols;
+    const size_t lds = sizeof(cf32) * NC * (size_t)ct_col_ld(CTN1) + sizeof(float) * 8;
+    ProfScope prof(name, st);
+    hipLaunchKernelGGL((k_big_cols<BATCH, CTN1>), dim3((bp.n2 + NC - 1) / NC, nbatch), dim3(ct_col_threads(CTN1)), lds,
+                       st, a, bp.n1, bp.n2, bp.p1, twc, bp.twN, jb);
+    FPCC_CHECK(hipGetLastError());
+    return 0;
+}
+
 template <bool BATCH>
 static int launch_cols(const BigPlan &bp, const ColArgs &a, const RealBatch &jb, int nbatch, hipStream_t st,
                        const char *name)
 {
-    const dim3 grid((bp.n2 + kBigCols - 1) / kBigCols, nbatch);
-    if (bp.n1 == kCtN1) {  // compile-time in-place column transform, one LDS buffer
-        const cf32 *twc = (const cf32 *)get_order_twiddles(kCtN1, {16, 16});
-        if (!twc) return -1;
-        const size_t lds = sizeof(cf32) * kBigCols * (size_t)kCtLD + sizeof(float) * 8;
-        ProfScope prof(name, st);
-        hipLaunchKernelGGL((k_big_cols<BATCH, true>), grid, dim3(256), lds, st, a, bp.n1, bp.n2, bp.p1, twc, bp.twN,
-                           jb);
-    } else {
-        const size_t lds = sizeof(cf32) * 2 * kBigCols * (size_t)(bp.n1 + 1) + sizeof(float) * 8;
-        allow_lds((const void *)k_big_cols<BATCH, false>, lds);
-        ProfScope prof(name, st);
-        hipLaunchKernelGGL((k_big_cols<BATCH, false>), grid, dim3(256), lds, st, a, bp.n1, bp.n2, bp.p1, bp.tw1,
-                           bp.twN, jb);
+    switch (bp.n1) {
+    case 256: return launch_cols_ct<BATCH, 256>(bp, a, jb, nbatch, st, name);
+    case 128: return launch_cols_ct<BATCH, 128>(bp, a, jb, nbatch, st, name);
+    case 64:
+        if (a.op != COL_INV_LAGWIN) return launch_cols_ct<BATCH, 64>(bp, a, jb, nbatch, st, name);
+        break;
+    case 32:
+        if (a.op != COL_INV_LAGWIN) return launch_cols_ct<BATCH, 32>(bp, a, jb, nbatch, st, name);
+        break;
     }
+    const dim3 grid((bp.n2 + kBigCols - 1) / kBigCols, nbatch);
+    const size_t lds = sizeof(cf32) * 2 * kBigCols * (size_t)(bp.n1 + 1) + sizeof(float) * 8;
+    allow_lds((const void *)k_big_cols<BATCH, 0>, lds);
+    ProfScope prof(name, st);
+    hipLaunchKernelGGL((k_big_cols<BATCH, 0>), grid, dim3(256), lds, st, a, bp.n1, bp.n2, bp.p1, bp.tw1, bp.twN, jb);
     FPCC_CHECK(hipGetLastError());
     return 0;
 }

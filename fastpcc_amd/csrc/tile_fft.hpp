@@ -20,15 +20,15 @@ __device__ __forceinline__ cf32 tw_m(const cf32 *__restrict__ twN, unsigned m)
 // (8 x 8 x 8, stride 544) or 4 x 1024 (16 x 8 x 8, stride 1088).  The strides keep
 // the loads, passes and stores within 1.5x of conflict-free LDS access.
 
-template <int NPT, int NTR, int LDT, int DIR, int R, int NS>
+template <int NPT, int NTR, int LDT, int DIR, int R, int NS, int NT = 256>
 __device__ __forceinline__ void ctb_pass(cf32 *lds, const cf32 *__restrict__ tw)
 {
-    constexpr int NBF = NPT / R, TOT = NTR * NBF, BPT = (TOT + 255) / 256;
+    constexpr int NBF = NPT / R, TOT = NTR * NBF, BPT = (TOT + NT - 1) / NT;
     cf32 v[BPT][R];
 #pragma unroll
     for (int i = 0; i < BPT; ++i) {
-        const int bb = threadIdx.x + 256 * i;
-        if (TOT % 256 == 0 || bb < TOT) {
+        const int bb = threadIdx.x + NT * i;
+        if (TOT % NT == 0 || bb < TOT) {
             const int t = bb / NBF, b = bb % NBF;
 #pragma unroll
             for (int r = 0; r < R; ++r) v[i][r] = lds[t * LDT + ct_pad(b + r * NBF)];
@@ -37,8 +37,8 @@ __device__ __forceinline__ void ctb_pass(cf32 *lds, const cf32 *__restrict__ tw)
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < BPT; ++i) {
-        const int bb = threadIdx.x + 256 * i;
-        if (TOT % 256 == 0 || bb < TOT) {
+        const int bb = threadIdx.x + NT * i;
+        if (TOT % NT == 0 || bb < TOT) {
             const int t = bb / NBF, b = bb % NBF;
             const int k = b % NS;
             if (NS > 1) {
@@ -85,11 +85,11 @@ __device__ __forceinline__ void ctb_last_regs(const cf32 *lds, int t, int b, cf3
     Dft<R, DIR>::run(v);
 }
 
-template <int NPT, int NTR, int LDT, int DIR, int NS, int OFF, int R, int... Rest>
+template <int NT, int NPT, int NTR, int LDT, int DIR, int NS, int OFF, int R, int... Rest>
 __device__ __forceinline__ void ctb_passes(cf32 *lds, const cf32 *__restrict__ tw)
 {
-    ctb_pass<NPT, NTR, LDT, DIR, R, NS>(lds, tw + OFF);
-    if constexpr (sizeof...(Rest) > 0) ctb_passes<NPT, NTR, LDT, DIR, NS * R, OFF + (R - 1) * NS, Rest...>(lds, tw);
+    ctb_pass<NPT, NTR, LDT, DIR, R, NS, NT>(lds, tw + OFF);
+    if constexpr (sizeof...(Rest) > 0) ctb_passes<NT, NPT, NTR, LDT, DIR, NS * R, OFF + (R - 1) * NS, Rest...>(lds, tw);
 }
 
 // tw: the per-pass twiddles of the plan with radices Rs (in that order)
@@ -97,7 +97,7 @@ template <int NPT, int NTR, int LDT, int DIR, int... Rs>
 __device__ __forceinline__ cf32 *ctb_fft(cf32 *lds, const cf32 *__restrict__ tw)
 {
     static_assert((Rs * ... * 1) == NPT, "radices must multiply to NPT");
-    ctb_passes<NPT, NTR, LDT, DIR, 1, 0, Rs...>(lds, tw);
+    ctb_passes<256, NPT, NTR, LDT, DIR, 1, 0, Rs...>(lds, tw);
     return lds;
 }
 
