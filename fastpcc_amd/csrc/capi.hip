@@ -702,8 +702,7 @@ int pair_stage(const fpcc_job *job, const Dims &d, char *ws, size_t ws_bytes, fl
         if (job->stack == FPCC_STACK_PWS)  // the reference's 1/((float)Nz*(float)N) of each window
             return launch_pair_pws(0, ws + l.a, nullptr, d.Nz, d.S, d.W, (int)d.Nz, d.lag0, d.L,
                                    1 / ((float)d.Nz * (float)d.N), (float)job->pws_power, 0, y, st);
-        return launch_pair_pcc2((const cf32 *)(ws + l.a), d.S, d.W, d.N, d.Nz, d.lag0, d.L, job->stack, 0,
-                                (int)d.P, y, st);
+        return launch_pair_pcc2((const cf32 *)(ws + l.a), d.S, d.W, d.N, d.Nz, d.lag0, d.L, job->stack, y, st);
     case FPCC_GNCC:
         r = launch_pair_gn(ws + l.a, ws + l.a, (const double *)(ws + l.b), true, d.S, d.W, d.N, d.Nz, d.lag0, d.L, 0,
                            mode, y, st);

@@ -179,8 +179,7 @@ k_pair_gn(const C2<T> *__restrict__ Xa, const C2<T> *__restrict__ Xb, long long 
     // the bins it folds, t + 512 q, from registers, and its last one gives the
     // transform values t and t + 3584 (lags 2t, 2t + 1 and 2t - 1024, 2t - 1023),
     // normalised and summed over the windows in registers
-    // (FP64 only: the FP32 kernel keeps four waves a SIMD only without it)
-    constexpr bool kRegs = CT4096 && sizeof(T) == 8;
+    constexpr bool kRegs = CT4096;
     const bool ends = kRegs && lag0 >= -1024 && lag0 + L - 1 <= 1023;
     float ar[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (!ends)
@@ -347,6 +346,9 @@ int launch_pair_gn(const void *d_Xa, const void *d_Xb, const double *d_E, bool f
                    int lag0, int L, int norm, int mode, float *d_y, hipStream_t st, const float *d_edge)
 {
     const int K = d_edge ? edge_len(N) : 0;
+    if (!f64 && norm == 1 && pair_short_ok(Nz))
+        return launch_short_1bit((const cf32 *)d_Xa, (const cf32 *)d_Xb, real_ld(Nz), S, W, N, Nz, lag0, L, mode, d_y, d_edge,
+                                 st);
     const int M = Nz / 2;
     const DevPlan &pM = get_plan(M, f64);
     const void *twc = get_c2r_twiddles(Nz, f64);
@@ -356,7 +358,7 @@ int launch_pair_gn(const void *d_Xa, const void *d_Xb, const double *d_E, bool f
     if (!blocks) return 0;
     const size_t elem = f64 ? sizeof(cf64) : sizeof(cf32);
     // Nz 8192: the compile-time in-place inverse and its own twiddle order
-    const bool ct = M == 4096;
+    const bool ct = f64 && M == 4096;
     const void *tw = ct ? get_order_twiddles(M, {8, 8, 8, 8}, f64) : pM.tw;
     if (!tw) return -1;
     size_t lds = elem * (ct ? (size_t)ct_lds_elems<4096>() : 2 * (size_t)M) + sizeof(float) * (size_t)L;
@@ -372,7 +374,7 @@ int launch_pair_gn(const void *d_Xa, const void *d_Xb, const double *d_E, bool f
                            real_ld(Nz), d_E, energy_ld(N), S, W, N, Nz, pM.plan, (const cf64 *)tw,
                            (const cf64 *)twc, lag0, L, norm, mode, d_y, d_edge, K, GnBatch{});
     } else {
-        const auto fn = ct ? k_pair_gn<float, true, false> : k_pair_gn<float, false, false>;
+        const auto fn = k_pair_gn<float, false, false>;
         allow_lds((const void *)fn, lds);
         hipLaunchKernelGGL(fn, dim3(blocks), dim3(512), lds, st, (const cf32 *)d_Xa, (const cf32 *)d_Xb,
                            real_ld(Nz), d_E, energy_ld(N), S, W, N, Nz, pM.plan, (const cf32 *)tw,
@@ -402,8 +404,10 @@ int launch_pair_gn_batch(GnBatch jb, bool f64, int Nz, int norm, int mode, hipSt
     if (blocks > 0x7fffffff) return -1;
     jb.b0[jb.n] = (int)blocks;
     if (!blocks) return 0;
+    if (!f64 && norm == 1 && pair_short_ok(Nz))
+        return launch_short_1bit_batch(jb, (int)blocks, real_ld(Nz), Nz, mode, st);
     const size_t elem = f64 ? sizeof(cf64) : sizeof(cf32);
-    const bool ct = M == 4096;
+    const bool ct = f64 && M == 4096;
     const void *tw = ct ? get_order_twiddles(M, {8, 8, 8, 8}, f64) : pM.tw;
     if (!tw) return -1;
     size_t lds = elem * (ct ? (size_t)ct_lds_elems<4096>() : 2 * (size_t)M) + sizeof(float) * (size_t)Lmax;
@@ -417,7 +421,7 @@ int launch_pair_gn_batch(GnBatch jb, bool f64, int Nz, int norm, int mode, hipSt
                            (const cf64 *)tw, (const cf64 *)twc, 0, 0, norm, mode, (float *)nullptr,
                            (const float *)nullptr, 0, jb);
     } else {
-        const auto fn = ct ? k_pair_gn<float, true, true> : k_pair_gn<float, false, true>;
+        const auto fn = k_pair_gn<float, false, true>;
         allow_lds((const void *)fn, lds);
         hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(512), lds, st, (const cf32 *)nullptr,
                            (const cf32 *)nullptr, real_ld(Nz), (const double *)nullptr, 0LL, 0, 0, 0, Nz, pM.plan,

@@ -950,8 +950,8 @@ k_pair_c2r_4096(const cf32 *__restrict__ G, GLayout gl, int P, const cf32 *__res
 // k, Nz-k, M-k and M+k of both stations' spectra, folds it into the half-length
 // spectrum in registers as it writes LDS, and runs the radix-8^4 inverse; the
 // next window's bins load while the current one transforms.  MODE 0 writes every
-// window's lags, MODE 1 the mean of the windows' lags (accumulated in registers),
-// MODE 2 sums the folded spectra over the windows and transforms once a pair.
+// window's lags (few pairs: G units a pair, each a run of its windows), MODE 2 sums the
+// folded spectra over the windows and transforms once a pair.
 // One complex bin through a buffer resource at a byte offset (0 beyond the row).
 // The 64-bit result is reinterpreted whole: taking its two 32-bit lanes apart
 // compiled to one dword load read twice.
@@ -960,9 +960,9 @@ __device__ __forceinline__ cf32 ld_bin(__amdgpu_buffer_rsrc_t r, unsigned off)
     return __builtin_bit_cast(cf32, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
 }
 
-template <int NT, int LPT, int MODE, bool ENDS, bool BATCH>
+template <int NT, int MODE, bool ENDS, bool BATCH>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4)))
-k_pair_plain_4096(const cf32 *__restrict__ F, int S, int W, int P, const int *__restrict__ order,
+k_pair_plain_4096(const cf32 *__restrict__ F, int S, int W, int P, int G, const int *__restrict__ order,
                   const cf32 *__restrict__ twM, const cf32 *__restrict__ twc, int lag0, int L, float scale,
                   float *__restrict__ y, PlainBatch jb)
 {
@@ -974,8 +974,12 @@ k_pair_plain_4096(const cf32 *__restrict__ F, int S, int W, int P, const int *__
     const int t = threadIdx.x;
     const cf32 w0 = twc[t];  // twc[k] = exp(2 pi i k / Nz); twc[t + NT q] = w0 twc[NT q]
     cf32 sa[MODE == 2 ? H : 1], sc[MODE == 2 ? H : 1], sph = cf32{0.f, 0.f};
-    float acc[LPT];
-    for (int u = blockIdx.x; u < P; u += gridDim.x) {
+    for (int ug = blockIdx.x; ug < P * G; ug += gridDim.x) {
+        int u = ug, part = 0;
+        if (MODE == 0 && G > 1) {  // (the divisions cost the smallest jobs 1%)
+            u = ug / G;
+            part = ug - u * G;
+        }
         int uj = u;
         if (BATCH) {  // job j's pairs are u0[j] <= u < u0[j+1]: its spectra, order, lags and output
             int j = 0;
@@ -998,9 +1002,12 @@ k_pair_plain_4096(const cf32 *__restrict__ F, int S, int W, int P, const int *__
         // uniform across the workgroup: scalar registers hold the row addresses
         i = __builtin_amdgcn_readfirstlane(i);
         j = __builtin_amdgcn_readfirstlane(j);
-#pragma unroll
-        for (int q = 0; q < LPT; ++q) acc[q] = 0.f;
-        for (int w = 0; w < W; ++w) {
+        int wa = 0, wb = W;
+        if (MODE == 0 && G > 1) {
+            wa = (int)((long long)part * W / G);
+            wb = (int)((long long)(part + 1) * W / G);
+        }
+        for (int w = wa; w < wb; ++w) {
             // the two rows as buffer resources (scalar registers) read at 32-bit lane
             // offsets: plain pointers with lane indices made the compiler keep one
             // 64-bit address per load across the loop and spill
@@ -1061,23 +1068,10 @@ k_pair_plain_4096(const cf32 *__restrict__ F, int S, int W, int P, const int *__
             if (ENDS) ct_last_pass_ends_4096(alt, lds, tw + 7 + 56 + 448);
             else ct_pass_oop<float, M, NT, +1, 8, 512, 0, 0>(alt, lds, tw + 7 + 56 + 448);
             float *dst = y + (MODE == 0 ? ((long long)p * W + w) * L : (long long)p * L);
-#pragma unroll
-            for (int q = 0; q < LPT; ++q) {
-                const int l = t + NT * q;
-                if (l < L) {
-                    const int n = (lag0 + l) & (Nz - 1);
-                    const cf32 v = lds[n >> 1];
-                    const float val = scale * ((n & 1) ? v.y : v.x);
-                    if (MODE == 1) acc[q] += val;
-                    else dst[l] = val;
-                }
-            }
-            if (MODE == 1 && w + 1 == W) {
-#pragma unroll
-                for (int q = 0; q < LPT; ++q) {
-                    const int l = t + NT * q;
-                    if (l < L) dst[l] = acc[q] / (float)W;
-                }
+            for (int l = t; l < L; l += NT) {
+                const int n = (lag0 + l) & (Nz - 1);
+                const cf32 v = lds[n >> 1];
+                dst[l] = scale * ((n & 1) ? v.y : v.x);
             }
             // the next fold writes the buffer the last pass read (every lane is past
             // that pass's barrier); these outputs are read before the next
@@ -1330,16 +1324,16 @@ static int launch_c2r_4096(const cf32 *d_G, const GLayout &gl, int P, const cf32
     return 0;
 }
 
-template <int LPT, int MODE, bool ENDS>
-static int launch_plain_4096_t(const cf32 *d_F, int S, int W, int P, const cf32 *twr, const cf32 *twc, int lag0,
-                               int L, float scale, float *d_y, hipStream_t st, const char *name)
+// Workgroups of the pair kernel that run at once, and the units a pair's windows are
+// split into when the pairs alone (MODE 0) do not fill them: one pair of 24 windows took
+// 119 us on one workgroup, 11 us on 24.
+template <int MODE, bool ENDS, bool BATCH>
+static int launch_plain_4096_t(const cf32 *d_F, int S, int W, int P, const int *order, const cf32 *twr, const cf32 *twc,
+                               int lag0, int L, float scale, float *d_y, const PlainBatch &jb, hipStream_t st,
+                               const char *name)
 {
-    // tiles of 16 stations: two tiles' spectra (32 stations x W windows x 64 KB, 49 MB
-    // at W 24) cover the pairs the resident workgroups run at once
-    const int *order = pair_tile_order(S, 16);
-    if (!order) return -1;
     constexpr int kT = kC2rThreads;
-    const auto fn = k_pair_plain_4096<kT, LPT, MODE, ENDS, false>;
+    const auto fn = k_pair_plain_4096<kT, MODE, ENDS, BATCH>;
     const size_t lds = sizeof(cf32) * 2 * 4096;
     int dev = 0, ncu = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
@@ -1352,113 +1346,60 @@ static int launch_plain_4096_t(const cf32 *d_F, int S, int W, int P, const cf32 
             per_cu = 1;
         per_cu_cached.store(per_cu, std::memory_order_relaxed);
     }
-    const int nwg = P < per_cu * ncu ? P : per_cu * ncu;
+    const int slots = per_cu * ncu;
+    const int G = MODE == 0 ? std::max(1, std::min(W, slots / P)) : 1;  // G > 1: P G <= slots
+    const int nwg = P * G < slots ? P * G : slots;
     ProfScope prof(name, st);
-    hipLaunchKernelGGL(fn, dim3(nwg), dim3(kT), lds, st, d_F, S, W, P, order, twr, twc, lag0, L, scale, d_y,
-                       PlainBatch{});
+    hipLaunchKernelGGL(fn, dim3(nwg), dim3(kT), lds, st, d_F, S, W, P, G, order, twr, twc, lag0, L, scale, d_y, jb);
     FPCC_CHECK(hipGetLastError());
     return 0;
 }
 
-template <int MODE>
-static int launch_plain_4096_m(int lpt, const cf32 *d_F, int S, int W, int P, const cf32 *twr, const cf32 *twc,
-                               int lag0, int L, float scale, float *d_y, hipStream_t st, const char *name)
-{
-    // lags within +-1024: the last pass forms only the outputs they read
-    const bool ends = lag0 >= -1024 && lag0 + L - 1 <= 1023;
-#define FPCC_PLAIN(LPT, E) launch_plain_4096_t<LPT, MODE, E>(d_F, S, W, P, twr, twc, lag0, L, scale, d_y, st, name)
-    switch (lpt) {
-    case 1: return ends ? FPCC_PLAIN(1, true) : FPCC_PLAIN(1, false);
-    case 2: return ends ? FPCC_PLAIN(2, true) : FPCC_PLAIN(2, false);
-    case 4: return ends ? FPCC_PLAIN(4, true) : FPCC_PLAIN(4, false);
-    case 8: return FPCC_PLAIN(8, false);
-    case 16: return FPCC_PLAIN(16, false);
-    }
-#undef FPCC_PLAIN
-    return -1;
-}
+// lags within +-1024: the last pass forms only the outputs they read
+static bool plain_ends(int lag0, int L) { return lag0 >= -1024 && lag0 + L - 1 <= 1023; }
 
+// mode 0: every window; else the mean over windows (one inverse of the summed spectra)
 int launch_pair_pcc2_4096(const cf32 *d_F, int S, int W, int N, int lag0, int L, int mode, float *d_y,
                           hipStream_t st)
 {
     constexpr int Nz = 8192;
     const long long P = (long long)S * (S - 1) / 2;
     if (P < 1 || P > 0x7fffffff || W < 1 || L < 1 || L > Nz || mode < 0 || mode > 2) return -1;
-    const void *twc = get_c2r_twiddles(Nz, false);
+    const cf32 *twc = (const cf32 *)get_c2r_twiddles(Nz, false);
     const cf32 *twr = (const cf32 *)get_order_twiddles(4096, {8, 8, 8, 8});
-    if (!twc || !twr) return -1;
-    int lpt = 1;
-    while (lpt * kC2rThreads < L) lpt *= 2;
+    // tiles of 16 stations: two tiles' spectra (32 stations x W windows x 64 KB, 49 MB
+    // at W 24) cover the pairs the resident workgroups run at once
+    const int *order = pair_tile_order(S, 16);
+    if (!twc || !twr || !order) return -1;
     // the folded spectra are twice the half spectrum of the real correlation: 1/2
-    // times the reference's 1/((float)Nz*(float)N) (mode 2 also takes the mean's 1/W)
+    // times the reference's 1/((float)Nz*(float)N) (the mean also takes 1/W)
     float scale = 0.5f * (1 / ((float)Nz * (float)N));
-    if (mode == 2) scale /= (float)W;
-    const cf32 *tc = (const cf32 *)twc;
-    switch (mode) {
-    case 0: return launch_plain_4096_m<0>(lpt, d_F, S, W, (int)P, twr, tc, lag0, L, scale, d_y, st, "pair_pcc2_none");
-    case 1: return launch_plain_4096_m<1>(lpt, d_F, S, W, (int)P, twr, tc, lag0, L, scale, d_y, st, "pair_pcc2_plain");
-    default: return launch_plain_4096_m<2>(lpt, d_F, S, W, (int)P, twr, tc, lag0, L, scale, d_y, st, "pair_pcc2_zsum");
-    }
+    if (mode) scale /= (float)W;
+    if (W == 1) mode = 0;  // one window is its own mean (the summing kernel keeps more registers)
+    const bool ends = plain_ends(lag0, L);
+#define FPCC_PLAIN(MODE, E, NAME)                                                                                  \
+    launch_plain_4096_t<MODE, E, false>(d_F, S, W, (int)P, order, twr, twc, lag0, L, scale, d_y, PlainBatch{}, st, NAME)
+    if (mode == 0) return ends ? FPCC_PLAIN(0, true, "pair_pcc2_none") : FPCC_PLAIN(0, false, "pair_pcc2_none");
+    return ends ? FPCC_PLAIN(2, true, "pair_pcc2_mean") : FPCC_PLAIN(2, false, "pair_pcc2_mean");
+#undef FPCC_PLAIN
 }
 
-// The per-window PCC2 pair stages of several jobs at Nz 8192 (one stack mode) in
-// one launch of the persistent pair kernel: a job table of spectra, station and
-// window counts, lag windows and outputs, the pairs of all jobs walked as one
-// sequence (each job's in its own tile order).
-template <int LPT, int MODE, bool ENDS>
-static int launch_plain_4096_batch_t(const PlainBatch &jb, int P, const cf32 *twr, const cf32 *twc, hipStream_t st)
-{
-    constexpr int kT = kC2rThreads;
-    const auto fn = k_pair_plain_4096<kT, LPT, MODE, ENDS, true>;
-    const size_t lds = sizeof(cf32) * 2 * 4096;
-    int dev = 0, ncu = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1)
-        return -1;
-    static std::atomic<int> per_cu_cached{0};
-    int per_cu = per_cu_cached.load(std::memory_order_relaxed);
-    if (!per_cu) {
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)fn, kT, lds) != hipSuccess || per_cu < 1)
-            per_cu = 1;
-        per_cu_cached.store(per_cu, std::memory_order_relaxed);
-    }
-    const int nwg = P < per_cu * ncu ? P : per_cu * ncu;
-    ProfScope prof(MODE == 0 ? "pair_pcc2_none_batch" : MODE == 1 ? "pair_pcc2_plain_batch" : "pair_pcc2_zsum_batch",
-                   st);
-    hipLaunchKernelGGL(fn, dim3(nwg), dim3(kT), lds, st, (const cf32 *)nullptr, 0, 0, P, (const int *)nullptr, twr,
-                       twc, 0, 0, 0.f, (float *)nullptr, jb);
-    FPCC_CHECK(hipGetLastError());
-    return 0;
-}
-
-template <int MODE>
-static int launch_plain_4096_batch_m(int lpt, bool ends, const PlainBatch &jb, int P, const cf32 *twr,
-                                     const cf32 *twc, hipStream_t st)
-{
-#define FPCC_PLAINB(LPT, E) launch_plain_4096_batch_t<LPT, MODE, E>(jb, P, twr, twc, st)
-    switch (lpt) {
-    case 1: return ends ? FPCC_PLAINB(1, true) : FPCC_PLAINB(1, false);
-    case 2: return ends ? FPCC_PLAINB(2, true) : FPCC_PLAINB(2, false);
-    case 4: return ends ? FPCC_PLAINB(4, true) : FPCC_PLAINB(4, false);
-    case 8: return FPCC_PLAINB(8, false);
-    case 16: return FPCC_PLAINB(16, false);
-    }
-#undef FPCC_PLAINB
-    return -1;
-}
-
+// The PCC2 pair stages of several jobs at Nz 8192 (one stack mode) in one launch of
+// the persistent pair kernel: a job table of spectra, station and window counts, lag
+// windows and outputs, the pairs of all jobs walked as one sequence (each job's in its
+// own tile order).
 int launch_pair_pcc2_4096_batch(int n, const cf32 *const *d_F, const int *S, const int *W, const int *N,
                                 const int *lag0, const int *L, int mode, float *const *d_y, hipStream_t st)
 {
     constexpr int Nz = 8192;
     if (n < 1 || n > kMaxBatchJobs || mode < 0 || mode > 2) return -1;
-    const void *twc = get_c2r_twiddles(Nz, false);
+    const cf32 *twc = (const cf32 *)get_c2r_twiddles(Nz, false);
     const cf32 *twr = (const cf32 *)get_order_twiddles(4096, {8, 8, 8, 8});
     if (!twc || !twr) return -1;
     PlainBatch jb{};
     jb.n = n;
     long long P = 0;
-    int Lmax = 1;
+    int Wmax = 1;
     bool ends = true;
     for (int j = 0; j < n; ++j) {
         const long long Pj = (long long)S[j] * (S[j] - 1) / 2;
@@ -1472,24 +1413,21 @@ int launch_pair_pcc2_4096_batch(int n, const cf32 *const *d_F, const int *S, con
         jb.W[j] = W[j];
         jb.lag0[j] = lag0[j];
         jb.L[j] = L[j];
-        // as launch_pair_pcc2_4096: 1/2 times 1/((float)Nz*(float)N), mode 2 also 1/W
+        // as launch_pair_pcc2_4096: 1/2 times 1/((float)Nz*(float)N), the mean also 1/W
         float sc = 0.5f * (1 / ((float)Nz * (float)N[j]));
-        if (mode == 2) sc /= (float)W[j];
+        if (mode) sc /= (float)W[j];
         jb.scale[j] = sc;
         jb.y[j] = d_y[j];
-        Lmax = std::max(Lmax, L[j]);
-        ends = ends && lag0[j] >= -1024 && lag0[j] + L[j] - 1 <= 1023;
+        Wmax = std::max(Wmax, W[j]);
+        ends = ends && plain_ends(lag0[j], L[j]);
     }
     if (P > 0x7fffffff) return -1;
     jb.u0[n] = (int)P;
-    int lpt = 1;
-    while (lpt * kC2rThreads < Lmax) lpt *= 2;
-    const cf32 *tc = (const cf32 *)twc;
-    switch (mode) {
-    case 0: return launch_plain_4096_batch_m<0>(lpt, ends, jb, (int)P, twr, tc, st);
-    case 1: return launch_plain_4096_batch_m<1>(lpt, ends, jb, (int)P, twr, tc, st);
-    default: return launch_plain_4096_batch_m<2>(lpt, ends, jb, (int)P, twr, tc, st);
-    }
+#define FPCC_PLAIN(MODE, E, NAME)                                                                                  \
+    launch_plain_4096_t<MODE, E, true>(nullptr, 0, Wmax, (int)P, nullptr, twr, twc, 0, 0, 0.f, nullptr, jb, st, NAME)
+    if (mode == 0) return ends ? FPCC_PLAIN(0, true, "pair_pcc2_none_batch") : FPCC_PLAIN(0, false, "pair_pcc2_none_batch");
+    return ends ? FPCC_PLAIN(2, true, "pair_pcc2_mean_batch") : FPCC_PLAIN(2, false, "pair_pcc2_mean_batch");
+#undef FPCC_PLAIN
 }
 
 int launch_pair_c2r(const cf32 *d_G, GLayout gl, int P, int Nz, int N, int W, int lag0, int L, float scale,
@@ -1516,6 +1454,8 @@ int launch_pair_c2r(const cf32 *d_G, GLayout gl, int P, int Nz, int N, int W, in
         return count_norm ? launch_c2r_4096<true>(d_G, gl, P, twr, (const cf32 *)twc, lag0, L, scale, N, d_y, ed, st)
                           : launch_c2r_4096<false>(d_G, gl, P, twr, (const cf32 *)twc, lag0, L, scale, N, d_y, ed, st);
     }
+    if (M < 4096 && pair_short_ok(Nz))
+        return launch_short_gram(d_G, gl, P, Nz, N, W, lag0, L, scale, count_norm, d_y, ed.edge, ed.K, S, st);
     size_t lds = sizeof(cf32) * 2 * (size_t)M;
     allow_lds((const void *)k_pair_c2r, lds);
     ProfScope prof("pair_c2r", st);

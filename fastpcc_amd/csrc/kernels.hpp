@@ -25,11 +25,10 @@ int launch_pcc_time(const cf32 *d_phi, int S, int W, int N, int lag_first, int L
 // bytes of `part` (partial sums of a split launch; 0: not split).  launch_pcc_time
 // with part == nullptr runs unsplit.
 size_t pcc_time_scratch(int S, int W, int N, int L, int mode);
-// PCC2 pair stage over pairs [pair_base, pair_base+npairs) of S stations.
-// mode 0: y[p][w][L]; 1: mean over windows of per-window IFFTs; 2: IFFT of the
-// window sum (same result by linearity).
-int launch_pair_pcc2(const cf32 *d_F, int S, int W, int N, int Nz, int lag0, int L, int mode, int pair_base,
-                     int npairs, float *d_y, hipStream_t st);
+// PCC2 pair stage of all pairs.  mode 0: y[p][w][L]; else y[p][L], the mean over windows
+// as one IFFT of the window sum (linear).
+int launch_pair_pcc2(const cf32 *d_F, int S, int W, int N, int Nz, int lag0, int L, int mode, float *d_y,
+                     hipStream_t st);
 
 // Phase-weighted stack over windows (pws.hip) for Nz <= 8192 (pws_supported).
 // src 0: PCC2 phasor spectra F[s*W+w][ld]; 1: FP32 half spectra (1-bit: Xa the
@@ -134,8 +133,8 @@ struct PlainBatch {
     float scale[kMaxBatchJobs];
     float *y[kMaxBatchJobs];
 };
-// The pair stages of n PCC2 jobs at Nz 8192 with one stack mode (0 none, 1 plain,
-// 2 zsum): spectra d_F[j] of S[j] stations x W[j] windows, window length N[j],
+// The pair stages of n PCC2 jobs at Nz 8192 with one stack mode (0 none,
+// 1 plain and 2 zsum: the mean over windows): spectra d_F[j] of S[j] stations x W[j] windows, window length N[j],
 // lags lag0[j] .. lag0[j] + L[j] - 1, output d_y[j]; the same results as
 // launch_pair_pcc2 per job.
 int launch_pair_pcc2_4096_batch(int n, const cf32 *const *d_F, const int *S, const int *W, const int *N,
@@ -176,6 +175,18 @@ struct GnBatch {
 // The pair stages of the jobs of jb in one launch, the same results as
 // launch_pair_gn per job.
 int launch_pair_gn_batch(GnBatch jb, bool f64, int Nz, int norm, int mode, hipStream_t st);
+
+// Pair stages at Nz = 512 .. 8192 on compile-time FP32 inverses (pairshort.hip): PCC2 (Nz
+// up to 4096; mode 0 every window, else the mean), 1-bit half spectra (one job, or the
+// jobs of jb with their unit offsets b0 and edge lengths K), Gram rows (Nz up to 4096).
+bool pair_short_ok(int Nz);
+int launch_short_pcc2(const cf32 *d_F, int S, int W, int N, int Nz, int lag0, int L, int mode, float *d_y,
+                      hipStream_t st);
+int launch_short_1bit(const cf32 *d_Xa, const cf32 *d_Xb, long long ld, int S, int W, int N, int Nz, int lag0, int L,
+                      int mode, float *d_y, const float *d_edge, hipStream_t st);
+int launch_short_1bit_batch(const GnBatch &jb, int units, long long ld, int Nz, int mode, hipStream_t st);
+int launch_short_gram(const cf32 *d_G, const GLayout &gl, int P, int Nz, int N, int W, int lag0, int L, float scale,
+                      int count, float *d_y, const float *d_edge, int K, int S, hipStream_t st);
 
 // Windows longer than one workgroup's LDS (large.hip).
 bool large_supported(int kind, int N, int Nz);

@@ -277,64 +277,49 @@ __device__ __forceinline__ float real_out(const cf32 *z, int n)
     return (n & 1) ? v.y : v.x;
 }
 
-// mode 0: per-window outputs y[p][w][L]; 1: mean of per-window IFFTs y[p][L];
-// 2: IFFT of the window-summed folded spectrum, y[p][L] (identical by linearity).
+// Nz without a compile-time inverse (under 512).  mode 0: per-window outputs y[p][w][L];
+// else the mean over windows, one IFFT of the window-summed folded spectrum, y[p][L].
 __global__ void __launch_bounds__(512)
 k_pair_pcc2(const cf32 *__restrict__ F, int S, int W, int Nz, FftPlan planM, const cf32 *__restrict__ twM,
-            const cf32 *__restrict__ twc, int lag0, int L, float scale, int mode, int pair_base,
+            const cf32 *__restrict__ twc, int lag0, int L, float scale, int mode,
             float *__restrict__ y)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int M = Nz >> 1;
     cf32 *buf0 = reinterpret_cast<cf32 *>(smem_raw);
     cf32 *buf1 = buf0 + M;
-    float *acc = reinterpret_cast<float *>(buf1 + M);
     int p, w0, w1;
     if (mode == 0) {
-        p = blockIdx.x / W + pair_base;
+        p = blockIdx.x / W;
         w0 = blockIdx.x % W;
         w1 = w0 + 1;
     } else {
-        p = blockIdx.x + pair_base;
+        p = blockIdx.x;
         w0 = 0;
         w1 = W;
     }
     int i, j;
     pair_index(p, S, i, j);
     const int T = blockDim.x;
-    if (mode == 2) {
+    if (mode != 0) {
         for (int w = w0; w < w1; ++w) {
             fold_cross(F + (long long)(i * W + w) * Nz, F + (long long)(j * W + w) * Nz, Nz, twc, buf0, w > w0);
             __syncthreads();
         }
         cf32 *z = fft_lds<float, +1>(buf0, buf1, planM, twM);
         const float sc = scale / (float)W;
-        float *dst = y + (long long)(p - pair_base) * L;
+        float *dst = y + (long long)p * L;
         for (int l = threadIdx.x; l < L; l += T) {
             int n = (lag0 + l) & (Nz - 1);
             dst[l] = sc * real_out(z, n);
         }
         return;
     }
-    for (int l = threadIdx.x; l < L; l += T) acc[l] = 0.0f;
-    for (int w = w0; w < w1; ++w) {
-        fold_cross(F + (long long)(i * W + w) * Nz, F + (long long)(j * W + w) * Nz, Nz, twc, buf0, false);
-        __syncthreads();
-        cf32 *z = fft_lds<float, +1>(buf0, buf1, planM, twM);
-        for (int l = threadIdx.x; l < L; l += T) {
-            int n = (lag0 + l) & (Nz - 1);
-            acc[l] += scale * real_out(z, n);
-        }
-        __syncthreads();
-    }
-    if (mode == 0) {
-        float *dst = y + ((long long)(p - pair_base) * W + w0) * L;
-        for (int l = threadIdx.x; l < L; l += T) dst[l] = acc[l];
-    } else {
-        const float inv = 1.0f / (float)W;
-        float *dst = y + (long long)(p - pair_base) * L;
-        for (int l = threadIdx.x; l < L; l += T) dst[l] = acc[l] * inv;
-    }
+    fold_cross(F + (long long)(i * W + w0) * Nz, F + (long long)(j * W + w0) * Nz, Nz, twc, buf0, false);
+    __syncthreads();
+    cf32 *z = fft_lds<float, +1>(buf0, buf1, planM, twM);
+    float *dst = y + ((long long)p * W + w0) * L;
+    for (int l = threadIdx.x; l < L; l += T) dst[l] = scale * real_out(z, (lag0 + l) & (Nz - 1));
 }
 
 // gfx950 workgroups may address up to 160 KB of LDS; opt in above 64 KB.
@@ -429,24 +414,23 @@ int launch_station_phasor(const float *d_x, long long station_stride, int S, int
     return 0;
 }
 
-int launch_pair_pcc2(const cf32 *d_F, int S, int W, int N, int Nz, int lag0, int L, int mode, int pair_base,
-                     int npairs, float *d_y, hipStream_t st)
+int launch_pair_pcc2(const cf32 *d_F, int S, int W, int N, int Nz, int lag0, int L, int mode, float *d_y,
+                     hipStream_t st)
 {
-    if (Nz == 8192 && pair_base == 0 && npairs == S * (S - 1) / 2)
-        return launch_pair_pcc2_4096(d_F, S, W, N, lag0, L, mode, d_y, st);
-    const int M = Nz / 2;
+    if (Nz == 8192) return launch_pair_pcc2_4096(d_F, S, W, N, lag0, L, mode, d_y, st);
+    if (pair_short_ok(Nz)) return launch_short_pcc2(d_F, S, W, N, Nz, lag0, L, mode, d_y, st);
+    const int M = Nz / 2, npairs = S * (S - 1) / 2;
     const DevPlan &pM = get_plan(M, false);
     const void *twc = get_c2r_twiddles(Nz, false);
     if (!pM.ok || !twc) return -1;
     const float scale = 1 / ((float)Nz * (float)N);
     const int threads = 512;
-    size_t lds = sizeof(cf32) * 2 * (size_t)M + sizeof(float) * (size_t)L;
+    const size_t lds = sizeof(cf32) * 2 * (size_t)M;
     int blocks = mode == 0 ? npairs * W : npairs;
     if (blocks == 0) return 0;
-    allow_lds((const void *)k_pair_pcc2, lds);
-    ProfScope prof(mode == 2 ? "pair_pcc2_zsum" : "pair_pcc2_plain", st);
+    ProfScope prof(mode ? "pair_pcc2_mean" : "pair_pcc2_none", st);
     hipLaunchKernelGGL(k_pair_pcc2, dim3(blocks), dim3(threads), lds, st, d_F, S, W, Nz, pM.plan,
-                       (const cf32 *)pM.tw, (const cf32 *)twc, lag0, L, scale, mode, pair_base, d_y);
+                       (const cf32 *)pM.tw, (const cf32 *)twc, lag0, L, scale, mode, d_y);
     FPCC_CHECK(hipGetLastError());
     return 0;
 }

@@ -137,7 +137,7 @@ int cuda_tspcc2_set_freq(float **y0, float **x01, float **x02, unsigned int N, u
 enum { FPCC_PCC2 = 0, FPCC_PCC1 = 1, FPCC_PCCV = 2, FPCC_GNCC = 3, FPCC_CC1B = 4, FPCC_WPCC = 5 };
 enum {
     FPCC_STACK_NONE = 0,  /* per-window outputs                                       */
-    FPCC_STACK_PLAIN = 1, /* mean of per-window correlations (one IFFT per pair-window) */
+    FPCC_STACK_PLAIN = 1, /* mean of per-window correlations (PCC2 and 1-bit: one IFFT of the summed spectra) */
     FPCC_STACK_ZSUM = 2,  /* sum of folded cross spectra over windows, one IFFT per pair */
     FPCC_STACK_GRAM = 3,  /* per-frequency Hermitian rank-W Gram (FP32 MFMA), one IFFT per pair */
     FPCC_STACK_GRAM16 = 4, /* the same Gram on FP16 MFMA with split hi+lo operands           */
