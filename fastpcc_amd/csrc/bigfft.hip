@@ -428,6 +428,61 @@ k_big_cols(ColArgs a, int N1, int N2, FftPlan p1, const cf32 *__restrict__ tw1, 
     }
 }
 
+// The scales' column passes of WPCC for columns of 256 points (col_ampnorm_fused): a
+// thread's 16 rows q + 16 i of a column are the inputs of its first radix-16 butterfly
+// and the outputs of its second, in either direction.  MAX: inverse, max|z|^2 alone;
+// else inverse, AmpNorm, forward, step twiddles, in place.  Reading the rows twice and
+// writing them once, against write + read of the analytic scales in between: 24
+// stations x 56 scales x 131072, 672 + 832 us as COL_INV_MAX and COL_FWD_AMPNORM of
+// k_big_cols, here 329 + 728 us (in k_big_cols itself the second transform took its
+// registers from 167 to 213, and both passes lost: 772 + 1077 us).
+template <bool BATCH, bool MAX>
+__global__ void __launch_bounds__(256)
+k_scale_cols(ColArgs a, int N2, const cf32 *__restrict__ tw1, const cf32 *__restrict__ twN, RealBatch jb)
+{
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    constexpr int LDC = ct_col_ld(256);
+    cf32 *lds = reinterpret_cast<cf32 *>(smem_raw);
+    float *red = reinterpret_cast<float *>(lds + kBigCols * LDC);
+    int b = blockIdx.y;
+    if (BATCH) {
+        const int j = batch_job(jb, b);
+        b -= jb.b0[j];
+        a.src = a.dst = (cf32 *)jb.X[j];
+        a.maxbuf = jb.mx[j];
+    }
+    const int t = threadIdx.x % kBigCols, q = threadIdx.x / kBigCols, c = blockIdx.x * kBigCols + t;
+    const cf32 *src = a.src + (long long)b * a.bstride + c;
+    cf32 v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = src[(q + 16 * i) * N2];
+    const float eps = MAX ? 0.f : 1e-6f * a.maxbuf[b];
+    ctb_first_regs<256, LDC, +1, 16>(v, t, q, lds);
+    __syncthreads();
+    ctb_last_regs<256, LDC, +1, 16>(lds, t, q, v, tw1 + 15);
+    if (MAX) {
+        float m = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) m = fmaxf(m, v[i].x * v[i].x + v[i].y * v[i].y);
+        m = block_max(m, red);
+        if (threadIdx.x == 0) atomicMax(reinterpret_cast<int *>(a.maxbuf + b), __float_as_int(m));
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const cf32 u = v[i];
+        const float rr = 1.0f / sqrtf(u.x * u.x + u.y * u.y + eps);
+        v[i] = __builtin_isnormal(rr) ? cf32{u.x * rr, u.y * rr} : cf32{0.f, 0.f};
+    }
+    __syncthreads();  // every inverse has read its columns
+    ctb_first_regs<256, LDC, -1, 16>(v, t, q, lds);
+    __syncthreads();
+    ctb_last_regs<256, LDC, -1, 16>(lds, t, q, v, tw1 + 15);
+    cf32 *dst = a.dst + (long long)b * a.bstride + c;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) dst[(q + 16 * i) * N2] = cmul(v[i], tw_cr(twN, c, q + 16 * i));  // W_n^{n2 k1}
+}
+
 // BATCH: the rows of job j's destination (in place, ROW_FWD_PLAIN only).
 // CTN2 = 512 or 1024: N2 = CTN2 transforms in place (ct_rows_fft, tw2 its
 // twiddles); 0: the runtime plan with ping-pong buffers.
@@ -795,6 +850,17 @@ template <bool BATCH>
 static int launch_cols(const BigPlan &bp, const ColArgs &a, const RealBatch &jb, int nbatch, hipStream_t st,
                        const char *name)
 {
+    if (a.op == COL_INV_AMPNORM_FWD || (a.op == COL_INV_MAX && a.max_only)) {
+        if (!col_ampnorm_fused(bp)) return -1;
+        const cf32 *twc = (const cf32 *)get_order_twiddles(256, {16, 16});
+        if (!twc) return -1;
+        const size_t lds = sizeof(cf32) * kBigCols * (size_t)ct_col_ld(256) + sizeof(float) * 8;
+        ProfScope prof(name, st);
+        const auto fn = a.op == COL_INV_MAX ? k_scale_cols<BATCH, true> : k_scale_cols<BATCH, false>;
+        hipLaunchKernelGGL(fn, dim3(bp.n2 / kBigCols, nbatch), dim3(256), lds, st, a, bp.n2, twc, bp.twN, jb);
+        FPCC_CHECK(hipGetLastError());
+        return 0;
+    }
     switch (bp.n1) {
     case 256: return launch_cols_ct<BATCH, 256>(bp, a, jb, nbatch, st, name);
     case 128: return launch_cols_ct<BATCH, 128>(bp, a, jb, nbatch, st, name);
@@ -831,7 +897,8 @@ int run_cols_batch(const BigPlan &bp, const ColArgs &a, const RealBatch &jb, hip
     const int nbatch = jb.b0[jb.n];
     if (nbatch <= 0) return 0;
     if (!bp.ok || nbatch > 65535) return -1;
-    if (a.op != COL_FWD_INPUT && a.op != COL_INV_MAX && a.op != COL_FWD_AMPNORM && a.op != COL_FWD_AMPNORMF)
+    if (a.op != COL_FWD_INPUT && a.op != COL_INV_MAX && a.op != COL_FWD_AMPNORM && a.op != COL_FWD_AMPNORMF &&
+        a.op != COL_INV_AMPNORM_FWD)
         return -1;
     return launch_cols<true>(bp, a, jb, nbatch, st, name);
 }

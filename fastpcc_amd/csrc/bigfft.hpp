@@ -35,6 +35,9 @@ enum ColOp {
     // w_m = exp(-i pi m^2 / N):
     COL_FWD_CHIRP = 6,       // x[g] * w_g (g < N), forward
     COL_CHIRP_MID = 7,       // inverse -> mask_g * conj(conv_g) (g < N) -> forward
+    // inverse -> AmpNorm (COL_FWD_AMPNORM's) -> forward, the columns staying in registers
+    // (columns of 256 points: col_ampnorm_fused), after a COL_INV_MAX that stores nothing
+    COL_INV_AMPNORM_FWD = 9,
     COL_INV_CHIRP_MAX = 8,   // inverse -> z_g = conj(w_g conv_g), g < N, into dst rows of dst_bstride; max|z|^2
 };
 
@@ -62,6 +65,7 @@ struct ColArgs {
     float in_scale = 1.f;
     // COL_INV_MAX writes, COL_FWD_AMPNORM(F) read max|z|^2 per batch
     float *maxbuf = nullptr;
+    int max_only = 0;  // COL_INV_MAX: the maximum alone, no output (col_ampnorm_fused plans)
     int nvalid = 0;  // COL_FWD_AMPNORMF: valid samples per src row
     // Bluestein ops: chirp table (N values), mask scale, output row stride
     const cf32 *chirp = nullptr;
@@ -102,6 +106,9 @@ struct RowArgs {
     const cf32 *F = nullptr, *F2 = nullptr;
     int Sst = 2, Wb = 1, wsel = 0, Wfull = 1, wsum = 0, pair0 = 0;  // pair p = pair0 + b / Wb
 };
+
+// True where the column pass of n = bp.n runs COL_INV_AMPNORM_FWD.
+inline bool col_ampnorm_fused(const BigPlan &bp) { return bp.n1 == 256 && bp.n2 % kBigCols == 0; }
 
 // Bluestein grid for an N-point DFT: the smallest power of two >= max(64, 2N-1).
 int bluestein_n(int N);

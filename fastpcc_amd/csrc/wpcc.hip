@@ -200,8 +200,12 @@ int wpcc_station_stage(const float *d_x, long long station_stride, int S, int W,
     ca.dst = B;
     ca.bstride = Nz;
     ca.maxbuf = mx;
+    // the maximum first, the inverse columns again with AmpNorm and the forward columns:
+    // the analytic scales never go to HBM (five transfers of the spectra instead of six)
+    const bool fused = col_ampnorm_fused(bp);
+    ca.max_only = fused;
     if ((r = run_cols(bp, ca, (int)nb, st, "wpcc_scale_inv_cols"))) return r;
-    ca.op = COL_FWD_AMPNORM;
+    ca.op = fused ? COL_INV_AMPNORM_FWD : COL_FWD_AMPNORM;
     if ((r = run_cols(bp, ca, (int)nb, st, "wpcc_ampnorm_cols"))) return r;
     ra = RowArgs{};
     ra.op = ROW_FWD_SCALE;
@@ -271,8 +275,10 @@ int wpcc_station_stage_batch(int n, const float *const *x, const long long *stri
     ca = ColArgs{};
     ca.op = COL_INV_MAX;
     ca.bstride = Nz;
+    const bool fused = col_ampnorm_fused(bp);  // as wpcc_station_stage
+    ca.max_only = fused;
     if ((r = run_cols_batch(bp, ca, js, st, "wpcc_scale_inv_cols_batch"))) return r;
-    ca.op = COL_FWD_AMPNORM;
+    ca.op = fused ? COL_INV_AMPNORM_FWD : COL_FWD_AMPNORM;
     if ((r = run_cols_batch(bp, ca, js, st, "wpcc_ampnorm_cols_batch"))) return r;
     ra = RowArgs{};
     ra.op = ROW_FWD_SCALE;
