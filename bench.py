@@ -10,7 +10,7 @@ of all 6144 station windows) + pair stage (all pair correlations, stacked).
 
 Prints one JSON line: pair-correlations/s (one (pair, window) correlation of L
 lags = one unit) with the stack on split-FP16 MFMA (FP32 accumulation), the
-FP32 Gram and the plain FP32 path (per pair-window IFFT) timed beside it,
+FP32 Gram and the plain FP32 path (per-pair sums of cross spectra, one IFFT a pair) timed beside it,
 per-kernel roofline of the dominant kernel from HIP events recorded inside the
 timed region, the oracle's CPU rate on a bounded sample, and a serving run: a
 Poisson stream of uneven all-pairs jobs (4-128 stations, 1800-86400 samples,
