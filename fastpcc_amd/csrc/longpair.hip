@@ -210,9 +210,11 @@ k_long_pair(LongArgs a)
         }
 }
 
-// Lags of item b from its shares' outputs, with the two-pass inverse's epilogue.
+// Lags of item b from its shares' outputs, with the two-pass inverse's epilogue.  f: what
+// one share's outputs are to the n-point inverse's value (1/2 where the fold holds twice
+// the half spectrum); not part of ca.scale, which the exact short overlaps take as well.
 __global__ void __launch_bounds__(256)
-k_long_lags(ColArgs ca, const cf32 *__restrict__ C, long long bstride, int H, int n, int G, int gstride, int A)
+k_long_lags(ColArgs ca, const cf32 *__restrict__ C, long long bstride, int H, int n, int G, int gstride, int A, float f)
 {
     const int l = blockIdx.x * 256 + threadIdx.x, b = blockIdx.y;
     if (l >= ca.L) return;
@@ -223,7 +225,7 @@ k_long_lags(ColArgs ca, const cf32 *__restrict__ C, long long bstride, int H, in
     const float *row = reinterpret_cast<const float *>(C + (long long)b * bstride + (A * H + m)) + (lag & 1);
     float v = 0.f;
     for (int s = 0; s < G; ++s) v += row[2LL * s * gstride];
-    lagwin_store(ca, p, w, i, j, n, l, v);
+    lagwin_store(ca, p, w, i, j, n, l, f * v);
 }
 
 namespace {
@@ -311,11 +313,10 @@ int run_long_pair(const BigPlan &bp, const RowArgs &ra, const ColArgs &ca, bool 
                                                                           : launch_lp<1024, 3>(a, src, blocks, st);
     }
     if (r) return r;
-    ColArgs c = ca;
-    if (!(src == LP_REAL)) c.scale *= 0.5f;  // the fold holds twice the half spectrum
+    const float f = src == LP_REAL ? 1.0f : 0.5f;
     ProfScope prof("long_lags", st);
-    hipLaunchKernelGGL(k_long_lags, dim3((ca.L + 255) / 256, nbatch), dim3(256), 0, st, c, (const cf32 *)a.dst, a.bstride, H,
-                       bp.n, a.G, a.upg * 4096, a.A);
+    hipLaunchKernelGGL(k_long_lags, dim3((ca.L + 255) / 256, nbatch), dim3(256), 0, st, ca, (const cf32 *)a.dst, a.bstride, H,
+                       bp.n, a.G, a.upg * 4096, a.A, f);
     FPCC_CHECK(hipGetLastError());
     return 0;
 }

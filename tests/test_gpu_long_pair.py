@@ -46,3 +46,11 @@ def test_gram_rows(fp, orc, kind, stack, lag1, lag2):
 def test_many_items_share_less(fp, orc):
     """Enough pair-windows that a workgroup takes several units of row pairs."""
     _case(fp, orc, "pcc2", "none", 12, 20, 12000, -100, 100)
+
+
+# every lag of the window: those of short overlap are exact sums over the record's ends,
+# normalised like the others (1-bit values are multiples of 1/overlap)
+@pytest.mark.parametrize("W", [1, 3])
+@pytest.mark.parametrize("stack", ["gram", "gram16"])
+def test_gram_rows_to_the_last_lag(fp, orc, stack, W):
+    _case(fp, orc, "cc1b", stack, 12, W, 5000, -4990, 4990)
