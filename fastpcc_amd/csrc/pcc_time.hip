@@ -39,7 +39,8 @@ namespace fpcc {
 // 2^(V log2 x)), about 1 ulp and a few ulp per term, as the reference's CUDA
 // engine compiles its terms (fast math); the correctly rounded library versions
 // cost several times more instructions.  Sums over N terms of either sign keep
-// the output within 1e-8 of the correctly rounded terms.  x^V for V <= 0 keeps powf.
+// the output within 1e-8 of the correctly rounded terms.  x^V for V <= 0 keeps powf
+// (k_pcc_direct).
 __device__ __forceinline__ float hw_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 __device__ __forceinline__ float hw_pow(float x, float V)
 {
@@ -51,7 +52,7 @@ typedef __bf16 b8v __attribute__((ext_vector_type(8)));
 typedef float f4v __attribute__((ext_vector_type(4)));
 typedef unsigned u4v __attribute__((ext_vector_type(4)));
 
-enum { PT_SQRT = 0, PT_SQUARE = 1, PT_HWPOW = 2, PT_POW = 3 };
+enum { PT_SQRT = 0, PT_SQUARE = 1, PT_HWPOW = 2, PT_POW = 3 };  // PT_POW: k_pcc_direct
 
 constexpr float kPtD = 2896.3093757400986f;  // (2^11.5 d)^2 <= |x|: corr(x) <= 2^-24
 
@@ -116,12 +117,9 @@ __device__ __forceinline__ void pt_tile(float (&acc)[16], f16v P, f16v Q, float 
             if constexpr (FN == PT_SQRT) {
                 P[r] = hw_sqrt(s);
                 Q[r] = hw_sqrt(u);
-            } else if constexpr (FN == PT_HWPOW) {
+            } else {
                 P[r] = hw_pow(s, V);
                 Q[r] = hw_pow(u, V);
-            } else {
-                P[r] = powf(s, V);
-                Q[r] = powf(u, V);
             }
         }
     };
@@ -180,7 +178,7 @@ struct PtSplit {
 // i, j < 32, walked down the diagonal n0 = nstart, nstart + 32, ...: its sums over
 // i - j = r belong to lag lagA + 32 c + r, so 4 TPW tiles cover 4 TPW - 1 bands of 32
 // lags.  Each chunk of samples is staged in LDS by components (out-of-range samples
-// as alpha = 0, whose terms are zero).  The 16 FP32 sums a lane are added along the
+// as alpha = 0, whose terms are zero for V > 0).  The 16 FP32 sums a lane are added along the
 // tile's diagonals in FP64 every 4 chunks (64 terms).
 // Two or three waves a SIMD asked for: within 256 registers the MFMA results land in
 // ordinary registers (else the compiler puts them in accumulation registers, three
@@ -370,6 +368,63 @@ k_pcc_time(const cf32 *__restrict__ phi, int S, int W, int N, int lag_first, int
     }
 }
 
+// x y - z w, within 1.5 ulp: 0 where x = z and y = w (or x = w and y = z)
+__device__ __forceinline__ float prod_diff(float x, float y, float z, float w)
+{
+    const float p = z * w, e = fmaf(-z, w, p);
+    return fmaf(x, y, -p) + e;
+}
+
+// V <= 0: the terms of samples outside the windows are not zero (0^V), and a term grows
+// without bound as a nears b or -b, so this kernel sums the overlap alone and forms P
+// and Q without cancellation (exactly 0 for a = -b and a = b: infinite terms).  One lag
+// a thread, 256 lags of one output row a workgroup; bound by powf.
+constexpr int kPdT = 256, kPdRun = 64;  // samples staged at a time, terms summed in FP32 before FP64
+
+__global__ void __launch_bounds__(kPdT)
+k_pcc_direct(const cf32 *__restrict__ phi, int S, int W, int N, int lag_first, int L, float V, double div, int mode,
+             int nblk, float *__restrict__ y, int out_ld, int out_off)
+{
+    __shared__ float4 s1[kPdT], s2[2 * kPdT - 1];  // x, y, 1 - |.|^2 of beta and alpha
+    const int t = threadIdx.x, lb = blockIdx.x % nblk, row = blockIdx.x / nblk;
+    const int p = mode == 0 ? row / W : row;
+    const int w0 = mode == 0 ? row - p * W : 0, w1 = mode == 0 ? w0 + 1 : W;
+    int i, j;
+    pair_index(p, S, i, j);
+    const int lagA = lag_first + lb * kPdT, lagB = min(lagA + kPdT - 1, lag_first + L - 1), lag = lagA + t;
+    const int n_lo = max(0, -lag), n_hi = lag <= lagB ? min(N, N - lag) : n_lo;
+    const int nstart = max(0, -lagB), nend = min(N, N - lagA);
+    auto sample = [](cf32 v) { return float4{v.x, v.y, pt_delta(v), 0.f}; };
+    double acc = 0.0;
+    for (int w = w0; w < w1; ++w) {
+        const cf32 *p1 = phi + (long long)(i * W + w) * N;
+        const cf32 *p2 = phi + (long long)(j * W + w) * N;
+        for (int n0 = nstart; n0 < nend; n0 += kPdT) {
+            __syncthreads();
+            if (n0 + t < N) s1[t] = sample(p1[n0 + t]);
+            for (int e = t; e < 2 * kPdT - 1; e += kPdT) {
+                const int m = n0 + lagA + e;
+                if (m >= 0 && m < N) s2[e] = sample(p2[m]);
+            }
+            __syncthreads();
+            const int lo = max(n_lo, n0) - n0, hi = min(n_hi, n0 + kPdT) - n0;
+            for (int e0 = lo; e0 < hi; e0 += kPdRun) {
+                float sum = 0.f;
+                for (int e = e0; e < min(e0 + kPdRun, hi); ++e) {
+                    const float4 b = s1[e], a = s2[e + t];
+                    const float P = 2.f * prod_diff(a.x, b.x, -a.y, b.y), Q = 2.f * prod_diff(a.y, b.x, a.x, b.y);
+                    const float d = a.z - b.z, dd = d * d;
+                    sum += powf(fmaf(P, P, dd), V) - powf(fmaf(Q, Q, dd), V);
+                }
+                acc += (double)sum;
+            }
+        }
+    }
+    if (lag > lagB) return;
+    const int count = max(0, min(N, N - lag) - max(0, -lag));
+    y[(long long)row * out_ld + out_off + lb * kPdT + t] = (float)(acc / (div * count));
+}
+
 // The G partial sums of every lag of a row, in order, normalised.
 __global__ void __launch_bounds__(256)
 k_pcc_time_sum(const double *__restrict__ part, int N, int lag_first, int L, int G, double div, float *__restrict__ y,
@@ -423,8 +478,7 @@ int launch_pt(int fn, const cf32 *d_phi, int S, int W, int N, int lag_first, int
     switch (fn) {
     case PT_SQRT: FPCC_PT(PT_SQRT); break;
     case PT_SQUARE: FPCC_PT(PT_SQUARE); break;
-    case PT_HWPOW: FPCC_PT(PT_HWPOW); break;
-    default: FPCC_PT(PT_POW); break;
+    default: FPCC_PT(PT_HWPOW); break;
     }
 #undef FPCC_PT
     FPCC_CHECK(hipGetLastError());
@@ -465,6 +519,14 @@ int launch_pcc_time(const cf32 *d_phi, int S, int W, int N, int lag_first, int L
     const double div = (pcc1 ? 2.0 : pow(2.0, (double)V)) * rw;
     ProfScope prof(pcc1 ? "pcc1_time" : "pccv_time", st);
     int r;
+    if (fn == PT_POW) {
+        const int nblk = (L + kPdT - 1) / kPdT;
+        if (rows * nblk > 0x7fffffff) return -1;
+        hipLaunchKernelGGL(k_pcc_direct, dim3((unsigned)(rows * nblk)), dim3(kPdT), 0, st, d_phi, S, W, N, lag_first, L, V,
+                           div, mode, nblk, d_y, out_ld, out_off);
+        FPCC_CHECK(hipGetLastError());
+        return 0;
+    }
     if (tpw == 4) r = launch_pt<4>(fn, d_phi, S, W, N, lag_first, L, V, div, mode, sp, blocks, d_y, out_ld, out_off, part, st);
     else r = launch_pt<2>(fn, d_phi, S, W, N, lag_first, L, V, div, mode, sp, blocks, d_y, out_ld, out_off, part, st);
     if (r || sp.G == 1) return r;

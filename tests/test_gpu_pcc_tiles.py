@@ -94,3 +94,69 @@ def test_workspace_without_the_split_scratch(fp, hip, stack):
     # FP64 sums of the same FP32 partial sums of at most 64 terms, cut at other samples
     assert np.abs(small - full).max() <= 2e-8
     assert run(need - 256)[0] == -1
+
+
+def _phasors(x, W, N):
+    """FP64 phasors [S][W][N] and a bound of the FP32 station stage's error in each: a window
+    of any length takes up to four transforms of 2048 points and more, 2^-24 sqrt(log2 n)
+    of the window's rms each, 4e-7 together, and no sample is off by more than three
+    times that over |z|; 1e-7 for the half-angle phasor's rounding."""
+    X = np.fft.fft(x.reshape(-1, W, N).astype(np.float64), axis=-1)
+    k = np.arange(N)
+    X[..., (k > 0) & (2 * k < N)] *= 2
+    X[..., 2 * k > N] = 0
+    z = np.fft.ifft(X, axis=-1)
+    mag = np.abs(z)
+    rms = np.sqrt((mag ** 2).mean(axis=-1, keepdims=True))
+    return z / (mag + 1e-6 * mag.max(axis=-1, keepdims=True)), 1.2e-6 * rms / mag + 1e-7
+
+
+@pytest.mark.parametrize("S,W,N,lag1,lag2,stack", [
+    (3, 1, 100, 7, 40, "none"), (3, 2, 100, -99, 99, "plain"), (2, 1, 512, -256, 255, "none"),
+    (2, 3, 1001, -300, 20, "none"), (4, 2, 777, 5, 520, "plain"), (2, 1, 9001, -3, 3, "none")])
+@pytest.mark.parametrize("v", [-0.5, -1.5, 0.0])
+def test_powers_that_are_not_positive(fp, orc, S, W, N, lag1, lag2, stack, v):
+    """Terms of samples outside the windows would be infinite, and the terms inside grow
+    without bound where two phasors are nearly equal or opposite."""
+    x = _records(S, W, N, 3 * N + W, "noise")
+    y = fp.allpairs(x, W, N, lag1, lag2, kind="pccv", stack=stack, v=v)
+    yr = orc.allpairs("pccv", x, W, N, lag1, lag2, stacked=stack != "none", f64=True, v=v)
+    assert np.isfinite(y).all()
+    # first-order bound of a term's error: |v| r^(v-1) times the phasors' error e, and the
+    # rounding of the terms and their sums (2^-21 of each); r kept from below by 2 e
+    ph, er = _phasors(x, W, N)
+    tol = np.zeros(y.shape).reshape(-1, W if stack == "none" else 1, y.shape[-1])
+    for p, (i, j) in enumerate((i, j) for i in range(S) for j in range(i + 1, S)):
+        for w in range(W):
+            for l, lag in enumerate(range(lag1, lag2 + 1)):
+                a, b = slice(max(0, lag), min(N, N + lag)), slice(max(0, -lag), min(N, N - lag))
+                e = er[j, w, a] + er[i, w, b]
+                for r in (np.abs(ph[j, w, a] + ph[i, w, b]), np.abs(ph[j, w, a] - ph[i, w, b])):
+                    r = np.maximum(r - e, e)
+                    t = (abs(v) * r ** (v - 1) * e + 2.0 ** -21 * r ** v).sum() / (2 ** (v / 2) * (N - abs(lag)))
+                    tol[p, w if stack == "none" else 0, l] += t if stack == "none" else t / W
+    err = np.abs(y - yr).reshape(tol.shape)
+    print(f"v {v} N {N}: max|gpu-fp64| {err.max():.2e}, at most {(err / tol).max():.2f} of the bound", flush=True)
+    assert (err <= tol).all()
+
+
+def test_equal_and_opposite_records_at_a_negative_power(fp, orc):
+    """0^v: the terms of equal records at lag 0 are -inf, of opposite ones +inf."""
+    W, N, v = 2, 333, -0.5
+    x = _records(3, W, N, 5, "noise")
+    x[1], x[2] = x[0], -x[0]
+    for stack in ("none", "plain"):
+        y = fp.allpairs(x, W, N, -4, 4, kind="pccv", stack=stack, v=v)
+        yr = orc.allpairs("pccv", x, W, N, -4, 4, stacked=stack != "none", f64=True, v=v)
+        inf = np.isinf(yr)
+        assert inf.any() and (np.isinf(y) == inf).all() and (y[inf] == yr[inf]).all()
+        assert np.isfinite(y[~inf]).all()
+
+
+def test_host_entry_at_a_negative_power(fp):
+    """pcc_set runs the same kernels."""
+    W, N, v = 3, 450, -1.0
+    x = _records(2, W, N, 9, "noise")
+    y = fp.pcc_set(*x.reshape(2, W, N), v, -30, 200)
+    assert np.isfinite(y).all()
+    assert np.array_equal(y, fp.allpairs(x, W, N, -30, 200, kind="pccv", stack="none", v=v)[0])
