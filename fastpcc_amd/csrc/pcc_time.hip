@@ -170,7 +170,7 @@ __host__ __device__ constexpr int pt_bands(int tpw) { return kPtWaves * tpw - 1;
 // averaged) are spread: G units, each a run of windows, or (ns > 1) one of ns equal
 // parts of one window's samples.
 struct PtSplit {
-    int G, ns, nblk;  // units a row, parts a window, lag blocks a row
+    int G, ns, nblk, lags;  // units a row, parts a window, lag blocks a row, lags a block
 };
 
 // Workgroup of 4 waves: one lag block of 32 (4 TPW - 1) lags of one unit.  Tile c
@@ -219,8 +219,8 @@ k_pcc_time(const cf32 *__restrict__ phi, int S, int W, int N, int lag_first, int
     }
     int i, j;
     pair_index(p, S, i, j);
-    const int lagA = lag_first + lb * 32 * pt_bands(TPW);
-    const int lagB = min(lagA + 32 * pt_bands(TPW) - 1, lag_first + L - 1);
+    const int lagA = lag_first + lb * sp.lags;
+    const int lagB = min(lagA + sp.lags - 1, lag_first + L - 1);
     const int Lb = lagB - lagA + 1;
     int nstart = max(0, -lagB), nend = min(N, N - lagA);
     if (sp.ns > 1) {
@@ -358,7 +358,7 @@ k_pcc_time(const cf32 *__restrict__ phi, int S, int W, int N, int lag_first, int
     for (int l = t; l < Lb; l += kT) {
         const int c = l >> 5, r = l & 31;
         const double sum = diag[c][31 + r] + (r ? diag[c + 1][r - 1] : 0.0);
-        const int gl = lb * 32 * pt_bands(TPW) + l;
+        const int gl = lb * sp.lags + l;
         if (sp.G > 1) {
             part[(long long)ru * L + gl] = sum;
         } else {
@@ -456,7 +456,11 @@ int pt_tpw(long long rows, int rw, int L)
 
 PtSplit pt_split(long long rows, int rw, int N, int L, int tpw)
 {
-    PtSplit s{1, 1, (L + 32 * pt_bands(tpw) - 1) / (32 * pt_bands(tpw))};
+    // blocks of equal bands: consecutive workgroups go to the XCDs in turn, so one short
+    // block among two or four left half the chip or a quarter idle (780 pairs x 24 windows
+    // of 1800, 481 lags: 8.7 ms as 480 + 1, 6.5 ms as 256 + 225)
+    const int bands = (L + 31) / 32, nblk = (bands + pt_bands(tpw) - 1) / pt_bands(tpw), per = (bands + nblk - 1) / nblk;
+    PtSplit s{1, 1, (bands + per - 1) / per, 32 * per};
     const long long want = (kPtFill + rows * s.nblk - 1) / (rows * s.nblk);
     if (want <= rw) {
         s.G = (int)want;

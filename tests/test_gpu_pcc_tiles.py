@@ -1,5 +1,5 @@
-"""Time-domain PCC1 / PCC-v where the tiled kernel can go wrong: lag blocks of 224 and
-480 lags (bands of 32), chunks of 512 samples, split and unsplit launches, and the
+"""Time-domain PCC1 / PCC-v where the tiled kernel can go wrong: lag blocks of up to 224
+and 480 lags (bands of 32, equal blocks), chunks of 512 samples, split and unsplit launches, and the
 records that decide between its two ways of summing PCC1's terms."""
 import ctypes
 
@@ -45,7 +45,8 @@ def _check(y, yr, N, lag1, lag2, tol=TOL):
     (2, 1, 511, 0, 0, "none"), (2, 1, 512, -16, 15, "none"), (2, 1, 513, -16, 16, "none"),
     (3, 2, 1025, -112, 111, "none"), (3, 2, 1024, -112, 112, "plain"), (2, 5, 1600, -240, 239, "plain"),
     (2, 1, 5003, -240, 240, "none"), (40, 24, 64, -31, 31, "none"), (40, 24, 64, -63, 63, "plain"),
-    (24, 8, 700, 37, 690, "plain"), (2, 1, 2, -1, 1, "none")])
+    (24, 8, 700, 37, 690, "plain"), (12, 12, 700, -240, 240, "plain"), (12, 12, 700, -320, 161, "none"),
+    (12, 8, 900, -480, 480, "plain"), (2, 1, 2, -1, 1, "none")])
 @pytest.mark.parametrize("kind,v", [("pcc1", 1.0), ("pccv", 2.0), ("pccv", 1.5)])
 def test_tile_edges(fp, orc, S, W, N, lag1, lag2, stack, kind, v):
     if N == 2 and kind == "pccv":
