@@ -375,54 +375,92 @@ __device__ __forceinline__ float prod_diff(float x, float y, float z, float w)
     return fmaf(x, y, -p) + e;
 }
 
-// V <= 0: the terms of samples outside the windows are not zero (0^V), and a term grows
-// without bound as a nears b or -b, so this kernel sums the overlap alone and forms P
-// and Q without cancellation (exactly 0 for a = -b and a = b: infinite terms).  One lag
-// a thread, 256 lags of one output row a workgroup; bound by powf.
-constexpr int kPdT = 256, kPdRun = 64;  // samples staged at a time, terms summed in FP32 before FP64
+// 256 lags of one output row a workgroup, one a thread, over the overlap alone: for launches
+// that the tiles' blocks of lags and chunks of samples do not fill (pt_direct_faster), and
+// for V <= 0, where the terms of samples outside the windows are not zero (0^V) and a term
+// grows without bound as a nears b or -b (P and Q without cancellation: exactly 0 for
+// a = -b and a = b).  Bound by the vector unit, 12 operations a term: 2.4 T PCC1 terms/s
+// (18720 pair-windows of 2000, 2001 lags) where the tiles reach 3.3, and 2.8 against 2.3
+// at 241 lags.  LDS rows of 8 and 4 bytes: as rows of 16 their reads were the bound (1.3x
+// the time at 241 lags); two lags a thread halved the reads but left most launches too
+// few waves (0.6 .. 0.9x).
+constexpr int kPdLags = 256, kPdChunk = 256, kPdRun = 64;  // terms summed in FP32 before FP64
 
-__global__ void __launch_bounds__(kPdT)
+template <int FN>
+__device__ __forceinline__ float pd_term(cf32 a, float ad, cf32 b, float bd, float V)
+{
+    // b holds 2 beta: P, Q as in the tiles
+    float P, Q;
+    if constexpr (FN == PT_POW) {
+        P = prod_diff(a.x, b.x, -a.y, b.y);
+        Q = prod_diff(a.y, b.x, a.x, b.y);
+    } else {
+        P = fmaf(a.x, b.x, a.y * b.y);
+        Q = fmaf(a.y, b.x, -(a.x * b.y));
+    }
+    if constexpr (FN == PT_SQUARE) return fmaf(P, P, -(Q * Q));
+    const float d = ad - bd, dd = d * d, s = fmaf(P, P, dd), u = fmaf(Q, Q, dd);
+    if constexpr (FN == PT_SQRT) return hw_sqrt(s) - hw_sqrt(u);
+    if constexpr (FN == PT_HWPOW) return hw_pow(s, V) - hw_pow(u, V);
+    return powf(s, V) - powf(u, V);
+}
+
+template <int FN>
+__global__ void __launch_bounds__(kPdLags)
 k_pcc_direct(const cf32 *__restrict__ phi, int S, int W, int N, int lag_first, int L, float V, double div, int mode,
              int nblk, float *__restrict__ y, int out_ld, int out_off)
 {
-    __shared__ float4 s1[kPdT], s2[2 * kPdT - 1];  // x, y, 1 - |.|^2 of beta and alpha
+    constexpr int kA = kPdChunk + kPdLags;
+    __shared__ cf32 sb[kPdChunk], sa[kA];    // 2 beta, alpha (0 outside the window)
+    __shared__ float db[kPdChunk], da[kA];   // 1 - |.|^2
     const int t = threadIdx.x, lb = blockIdx.x % nblk, row = blockIdx.x / nblk;
     const int p = mode == 0 ? row / W : row;
     const int w0 = mode == 0 ? row - p * W : 0, w1 = mode == 0 ? w0 + 1 : W;
     int i, j;
     pair_index(p, S, i, j);
-    const int lagA = lag_first + lb * kPdT, lagB = min(lagA + kPdT - 1, lag_first + L - 1), lag = lagA + t;
-    const int n_lo = max(0, -lag), n_hi = lag <= lagB ? min(N, N - lag) : n_lo;
+    const int lagA = lag_first + lb * kPdLags, lagB = min(lagA + kPdLags - 1, lag_first + L - 1), lag = lagA + t;
     const int nstart = max(0, -lagB), nend = min(N, N - lagA);
-    auto sample = [](cf32 v) { return float4{v.x, v.y, pt_delta(v), 0.f}; };
+    // samples this lag takes (V <= 0), or any lag of the wave: the others' terms are zero
+    int lo0 = max(0, -lag), hi0 = lag <= lagB ? min(N, N - lag) : lo0;
+    if constexpr (FN != PT_POW) {
+        const int wl = lagA + 64 * __builtin_amdgcn_readfirstlane(t >> 6);
+        lo0 = max(0, -min(wl + 63, lagB));
+        hi0 = wl <= lagB ? min(N, N - wl) : lo0;
+    }
     double acc = 0.0;
     for (int w = w0; w < w1; ++w) {
         const cf32 *p1 = phi + (long long)(i * W + w) * N;
         const cf32 *p2 = phi + (long long)(j * W + w) * N;
-        for (int n0 = nstart; n0 < nend; n0 += kPdT) {
+        for (int n0 = nstart; n0 < nend; n0 += kPdChunk) {
             __syncthreads();
-            if (n0 + t < N) s1[t] = sample(p1[n0 + t]);
-            for (int e = t; e < 2 * kPdT - 1; e += kPdT) {
+            const int nc = min(kPdChunk, nend - n0);
+            if (t < nc) {
+                const cf32 v = p1[n0 + t];
+                sb[t] = cf32{2.f * v.x, 2.f * v.y};
+                db[t] = pt_delta(v);
+            }
+            // lanes past lagB in a wave that holds it read on: up to the next 64 lags
+            const int na = nc + ((lagB - lagA) | 63);
+            for (int e = t; e < na; e += kPdLags) {
                 const int m = n0 + lagA + e;
-                if (m >= 0 && m < N) s2[e] = sample(p2[m]);
+                const cf32 v = m >= 0 && m < N ? p2[m] : cf32{0.f, 0.f};
+                sa[e] = v;
+                da[e] = pt_delta(v);
             }
             __syncthreads();
-            const int lo = max(n_lo, n0) - n0, hi = min(n_hi, n0 + kPdT) - n0;
+            const int lo = max(lo0 - n0, 0), hi = min(hi0 - n0, nc);
             for (int e0 = lo; e0 < hi; e0 += kPdRun) {
+                const int e1 = min(e0 + kPdRun, hi);
                 float sum = 0.f;
-                for (int e = e0; e < min(e0 + kPdRun, hi); ++e) {
-                    const float4 b = s1[e], a = s2[e + t];
-                    const float P = 2.f * prod_diff(a.x, b.x, -a.y, b.y), Q = 2.f * prod_diff(a.y, b.x, a.x, b.y);
-                    const float d = a.z - b.z, dd = d * d;
-                    sum += powf(fmaf(P, P, dd), V) - powf(fmaf(Q, Q, dd), V);
-                }
+#pragma unroll 8
+                for (int e = e0; e < e1; ++e) sum += pd_term<FN>(sa[e + t], da[e + t], sb[e], db[e], V);
                 acc += (double)sum;
             }
         }
     }
     if (lag > lagB) return;
     const int count = max(0, min(N, N - lag) - max(0, -lag));
-    y[(long long)row * out_ld + out_off + lb * kPdT + t] = (float)(acc / (div * count));
+    y[(long long)row * out_ld + out_off + lb * kPdLags + t] = (float)(acc / (div * count));
 }
 
 // The G partial sums of every lag of a row, in order, normalised.
@@ -469,6 +507,40 @@ PtSplit pt_split(long long rows, int rw, int N, int L, int tpw)
         s.G = rw * s.ns;
     }
     return s;
+}
+
+// Whether one lag a thread is faster than the tiles: both times in us from the launch's
+// shape.  Tiles: workgroups (two of TPW 4 or three of TPW 2 a CU run at once) of a fixed
+// cost and, per 32 samples, the staging and products of all tiles and the terms of those
+// that hold lags; a chip they do not fill runs them faster.  One lag a thread: the
+// vector work of its waves, or a lone wave's latency.  The constants are those that pick
+// the faster one in 220 measured launches (S 2 .. 100, W 1 .. 30, N 16 .. 4096, up to 2001
+// lags; at worst 1.06x of the faster one's time).  The tiles alone ran at 0.1x of this
+// kernel's speed for 18720 windows of 16, 0.65 .. 0.85x for as many of 600 .. 2000 and up
+// to 501 lags; this kernel at 0.1x of theirs for few long windows.
+bool pt_direct_faster(int fn, long long rows, int rw, int N, int lag_first, int L, int tpw, const PtSplit &sp)
+{
+    struct Cost {
+        double unit, step4, tile4, step2, tile2, wave, serial, group;
+    };
+    static constexpr Cost kSqrt{12, 1.0, 0.14, 0.28, 0.52, 6e-4, 0.060, 3.6e-4};
+    static constexpr Cost kPow{6.5, 0.3, 0.58, 0.25, 0.30, 7.6e-4, 0.056, 4.5e-4};
+    static constexpr Cost kSquare{9, 0.5, 0.06, 0.26, 0.09, 5.5e-4, 0.040, 2.7e-4};
+    const Cost &c = fn == PT_SQRT ? kSqrt : fn == PT_SQUARE ? kSquare : kPow;
+    // samples a lag takes of a window, on average
+    const double a = lag_first, b = lag_first + L - 1;
+    const double n = N - (a < 0 && b > 0 ? (a * a + b * b) / (2 * (b - a)) : std::abs(a + b) / 2);
+    // tiles
+    const double windows = sp.ns > 1 ? 1.0 : (double)rw / sp.G, steps = n / 32 / sp.ns;
+    const int tiles = std::min((std::min(L, sp.lags) + 62) / 32, kPtWaves * tpw), deep = (tiles + kPtWaves - 1) / kPtWaves;
+    const double rounds = (double)rows * sp.G * sp.nblk / (tpw == 4 ? 512 : 768);
+    const double turns = rounds <= 1 ? 0.6 : rounds < 3 ? std::ceil(rounds) : rounds + 0.5;
+    const double step = tpw == 4 ? c.step4 + c.tile4 * deep : c.step2 + c.tile2 * deep;
+    const double tiled = turns * (c.unit + windows * steps * step);
+    // one lag a thread: four-norm of the two bounds
+    const double work = rw * n / 32 * rows * (c.wave * ((L + 63) / 64) + c.group * ((L + kPdLags - 1) / kPdLags));
+    const double alone = rw * n * c.serial;
+    return std::sqrt(std::hypot(work * work, alone * alone)) < tiled;
 }
 
 template <int TPW>
@@ -521,13 +593,22 @@ int launch_pcc_time(const cf32 *d_phi, int S, int W, int N, int lag_first, int L
     const int fn = pcc1 || V == 0.5f ? PT_SQRT : V == 1.0f ? PT_SQUARE : V > 0.f ? PT_HWPOW : PT_POW;
     // per lag: sum / (2 count) (:276) or sum / (2^(v/2) count) (:334), over the windows of a row
     const double div = (pcc1 ? 2.0 : pow(2.0, (double)V)) * rw;
-    ProfScope prof(pcc1 ? "pcc1_time" : "pccv_time", st);
+    const bool direct = fn == PT_POW || pt_direct_faster(fn, rows, rw, N, lag_first, L, tpw, sp);
+    ProfScope prof(direct ? (pcc1 ? "pcc1_direct" : "pccv_direct") : pcc1 ? "pcc1_time" : "pccv_time", st);
     int r;
-    if (fn == PT_POW) {
-        const int nblk = (L + kPdT - 1) / kPdT;
+    if (direct) {
+        const int nblk = (L + kPdLags - 1) / kPdLags;
         if (rows * nblk > 0x7fffffff) return -1;
-        hipLaunchKernelGGL(k_pcc_direct, dim3((unsigned)(rows * nblk)), dim3(kPdT), 0, st, d_phi, S, W, N, lag_first, L, V,
-                           div, mode, nblk, d_y, out_ld, out_off);
+        const dim3 g((unsigned)(rows * nblk)), b(kPdLags);
+#define FPCC_PD(FN)                                                                                               \
+    hipLaunchKernelGGL(k_pcc_direct<FN>, g, b, 0, st, d_phi, S, W, N, lag_first, L, V, div, mode, nblk, d_y, out_ld, out_off)
+        switch (fn) {
+        case PT_SQRT: FPCC_PD(PT_SQRT); break;
+        case PT_SQUARE: FPCC_PD(PT_SQUARE); break;
+        case PT_HWPOW: FPCC_PD(PT_HWPOW); break;
+        default: FPCC_PD(PT_POW); break;
+        }
+#undef FPCC_PD
         FPCC_CHECK(hipGetLastError());
         return 0;
     }

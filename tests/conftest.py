@@ -76,3 +76,25 @@ def hip(fp):
     h = HipMem()
     yield h
     h.free()
+
+
+@pytest.fixture
+def launched(fp):
+    """launched(call): the call's result and the names of the kernels that it launched (the
+    library's own timing), for tests of one path of a dispatch."""
+    import ctypes
+    lib = fp._lib.lib()
+
+    def run(call):
+        names = ctypes.create_string_buffer(16384)
+        lib.fpcc_profile_reset()
+        lib.fpcc_profile_enable(1)
+        try:
+            y = call()
+            lib.fpcc_profile_report(names, len(names), None, None, 256)
+        finally:
+            lib.fpcc_profile_enable(0)
+            lib.fpcc_profile_reset()
+        return y, set(names.value.decode().split())
+
+    return run

@@ -1,6 +1,7 @@
 """Time-domain PCC1 / PCC-v where the tiled kernel can go wrong: lag blocks of up to 224
-and 480 lags (bands of 32, equal blocks), chunks of 512 samples, split and unsplit launches, and the
-records that decide between its two ways of summing PCC1's terms."""
+and 480 lags (bands of 32, equal blocks), chunks of 512 samples, split and unsplit
+launches, and the records that decide between its two ways of summing PCC1's terms; and
+the kernel of one lag a thread at its edges."""
 import ctypes
 
 import numpy as np
@@ -44,17 +45,41 @@ def _check(y, yr, N, lag1, lag2, tol=TOL):
 @pytest.mark.parametrize("S,W,N,lag1,lag2,stack", [
     (2, 1, 511, 0, 0, "none"), (2, 1, 512, -16, 15, "none"), (2, 1, 513, -16, 16, "none"),
     (3, 2, 1025, -112, 111, "none"), (3, 2, 1024, -112, 112, "plain"), (2, 5, 1600, -240, 239, "plain"),
-    (2, 1, 5003, -240, 240, "none"), (40, 24, 64, -31, 31, "none"), (40, 24, 64, -63, 63, "plain"),
-    (24, 8, 700, 37, 690, "plain"), (12, 12, 700, -240, 240, "plain"), (12, 12, 700, -320, 161, "none"),
-    (12, 8, 900, -480, 480, "plain"), (2, 1, 2, -1, 1, "none")])
+    (2, 1, 5003, -240, 240, "none"), (4, 8, 1700, 37, 690, "plain"), (12, 12, 700, -240, 240, "plain"),
+    (12, 8, 900, -480, 480, "plain")])
 @pytest.mark.parametrize("kind,v", [("pcc1", 1.0), ("pccv", 2.0), ("pccv", 1.5)])
-def test_tile_edges(fp, orc, S, W, N, lag1, lag2, stack, kind, v):
-    if N == 2 and kind == "pccv":
-        pytest.skip("one length of this kind is enough")
+def test_tile_edges(fp, orc, launched, S, W, N, lag1, lag2, stack, kind, v):
     x = _records(S, W, N, S * N + W, "noise")
-    y = fp.allpairs(x, W, N, lag1, lag2, kind=kind, stack=stack, v=v)
+    y, names = launched(lambda: fp.allpairs(x, W, N, lag1, lag2, kind=kind, stack=stack, v=v))
+    assert kind + "_time" in names and kind + "_direct" not in names
     yr = orc.allpairs(kind, x, W, N, lag1, lag2, stacked=stack != "none", f64=True, v=v)
     _check(y, yr, N, lag1, lag2)
+
+
+# one lag a thread: blocks of 256 lags in waves of 64, chunks of 256 samples in runs of 64
+@pytest.mark.parametrize("S,W,N,lag1,lag2,stack", [
+    (2, 1, 2, -1, 1, "none"), (40, 24, 64, -31, 31, "none"), (40, 24, 64, -63, 63, "plain"),
+    (30, 9, 65, -64, 64, "none"), (30, 9, 255, 0, 0, "none"), (24, 8, 256, -32, 31, "none"),
+    (24, 8, 257, -128, 127, "none"), (24, 8, 257, -128, 128, "none"), (24, 8, 320, 5, 261, "none"),
+    (30, 9, 513, -100, -60, "none"), (12, 12, 700, -320, 161, "none")])
+@pytest.mark.parametrize("kind,v", [("pcc1", 1.0), ("pccv", 2.0), ("pccv", 1.5)])
+def test_one_lag_a_thread(fp, orc, launched, S, W, N, lag1, lag2, stack, kind, v):
+    x = _records(S, W, N, S * N + W, "noise")
+    y, names = launched(lambda: fp.allpairs(x, W, N, lag1, lag2, kind=kind, stack=stack, v=v))
+    assert kind + "_direct" in names and kind + "_time" not in names
+    yr = orc.allpairs(kind, x, W, N, lag1, lag2, stacked=stack != "none", f64=True, v=v)
+    _check(y, yr, N, lag1, lag2)
+
+
+@pytest.mark.parametrize("what", ["event", "silent", "antiphase"])
+@pytest.mark.parametrize("kind,v", [("pcc1", 1.0), ("pccv", 1.5)])
+def test_records_one_lag_a_thread(fp, orc, launched, what, kind, v):
+    S, W, N = 24, 6, 600
+    x = _records(S, W, N, 7, what)
+    y, names = launched(lambda: fp.allpairs(x, W, N, -100, 100, kind=kind, stack="none", v=v))
+    assert kind + "_direct" in names
+    yr = orc.allpairs(kind, x, W, N, -100, 100, stacked=False, f64=True, v=v)
+    _check(y, yr, N, -100, 100, tol=TOL if what == "antiphase" else TOL_SHORT)  # as test_records_on_both_ways
 
 
 @pytest.mark.parametrize("what", ["event", "silent", "antiphase"])
