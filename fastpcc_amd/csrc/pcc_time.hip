@@ -157,7 +157,7 @@ __device__ __forceinline__ void pt_tile(float (&acc)[16], f16v P, f16v Q, float 
 #pragma unroll
     for (int g = 0; g < 4; ++g) roots(g);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = acc[r] + P[r] - Q[r];
+    for (int r = 0; r < 16; ++r) acc[r] += P[r] - Q[r];  // the small difference first
 }
 
 constexpr int kPtWaves = 4;
