@@ -170,7 +170,7 @@ __host__ __device__ constexpr int pt_bands(int tpw) { return kPtWaves * tpw - 1;
 // averaged) are spread: G units, each a run of windows, or (ns > 1) one of ns equal
 // parts of one window's samples.
 struct PtSplit {
-    int G, ns, nblk, lags;  // units a row, parts a window, lag blocks a row, lags a block
+    int G, ns, nblk;  // units a row, parts a window, lag blocks a row
 };
 
 // Workgroup of 4 waves: one lag block of 32 (4 TPW - 1) lags of one unit.  Tile c
@@ -200,8 +200,12 @@ k_pcc_time(const cf32 *__restrict__ phi, int S, int W, int N, int lag_first, int
     static_assert(sizeof(float) * kPtWaves * 32 * 33 <= sizeof(ac) && sizeof(double) * kTiles * 64 <= sizeof(bc), "fit");
     const int t = threadIdx.x, lane = t & 63, h = lane >> 5, lj = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int lb = blockIdx.x % sp.nblk;
     const int ru = blockIdx.x / sp.nblk, u = ru % sp.G, row = ru / sp.G;
+    // Workgroups go to the 8 XCDs in turn and the last lag block of a unit is short.  An even
+    // number of blocks would put it on the same XCDs in every unit (780 pairs x 24 windows of
+    // 1800, 481 lags: 8.7 ms, half the chip idle), so the blocks of a unit move on by one
+    // each time the pattern of units over XCDs repeats (7.3 ms).
+    const int g = sp.nblk & -sp.nblk, lb = (blockIdx.x % sp.nblk + (g > 1 ? ru / max(8 / g, 1) : 0)) % sp.nblk;
     const int p = mode == 0 ? row / W : row;
     // windows and sample range of this unit
     int w0, w1, part_i = 0;
@@ -219,8 +223,8 @@ k_pcc_time(const cf32 *__restrict__ phi, int S, int W, int N, int lag_first, int
     }
     int i, j;
     pair_index(p, S, i, j);
-    const int lagA = lag_first + lb * sp.lags;
-    const int lagB = min(lagA + sp.lags - 1, lag_first + L - 1);
+    const int lagA = lag_first + lb * 32 * pt_bands(TPW);
+    const int lagB = min(lagA + 32 * pt_bands(TPW) - 1, lag_first + L - 1);
     const int Lb = lagB - lagA + 1;
     int nstart = max(0, -lagB), nend = min(N, N - lagA);
     if (sp.ns > 1) {
@@ -358,7 +362,7 @@ k_pcc_time(const cf32 *__restrict__ phi, int S, int W, int N, int lag_first, int
     for (int l = t; l < Lb; l += kT) {
         const int c = l >> 5, r = l & 31;
         const double sum = diag[c][31 + r] + (r ? diag[c + 1][r - 1] : 0.0);
-        const int gl = lb * sp.lags + l;
+        const int gl = lb * 32 * pt_bands(TPW) + l;
         if (sp.G > 1) {
             part[(long long)ru * L + gl] = sum;
         } else {
@@ -494,11 +498,7 @@ int pt_tpw(long long rows, int rw, int L)
 
 PtSplit pt_split(long long rows, int rw, int N, int L, int tpw)
 {
-    // blocks of equal bands: consecutive workgroups go to the XCDs in turn, so one short
-    // block among two or four left half the chip or a quarter idle (780 pairs x 24 windows
-    // of 1800, 481 lags: 8.7 ms as 480 + 1, 6.5 ms as 256 + 225)
-    const int bands = (L + 31) / 32, nblk = (bands + pt_bands(tpw) - 1) / pt_bands(tpw), per = (bands + nblk - 1) / nblk;
-    PtSplit s{1, 1, (bands + per - 1) / per, 32 * per};
+    PtSplit s{1, 1, (L + 32 * pt_bands(tpw) - 1) / (32 * pt_bands(tpw))};
     const long long want = (kPtFill + rows * s.nblk - 1) / (rows * s.nblk);
     if (want <= rw) {
         s.G = (int)want;
@@ -514,8 +514,9 @@ PtSplit pt_split(long long rows, int rw, int N, int L, int tpw)
 // cost and, per 32 samples, the staging and products of all tiles and the terms of those
 // that hold lags; a chip they do not fill runs them faster.  One lag a thread: the
 // vector work of its waves, or a lone wave's latency.  The constants are those that pick
-// the faster one in 220 measured launches (S 2 .. 100, W 1 .. 30, N 16 .. 4096, up to 2001
-// lags; at worst 1.06x of the faster one's time).  The tiles alone ran at 0.1x of this
+// the faster one in 240 measured launches (S 2 .. 100, W 1 .. 30, N 16 .. 4096, up to 2001
+// lags; at worst 1.3x of the faster one's time, where the two are near each other and the
+// records decide how many roots the tiles take).  The tiles alone ran at 0.1x of this
 // kernel's speed for 18720 windows of 16, 0.65 .. 0.85x for as many of 600 .. 2000 and up
 // to 501 lags; this kernel at 0.1x of theirs for few long windows.
 bool pt_direct_faster(int fn, long long rows, int rw, int N, int lag_first, int L, int tpw, const PtSplit &sp)
@@ -523,7 +524,7 @@ bool pt_direct_faster(int fn, long long rows, int rw, int N, int lag_first, int 
     struct Cost {
         double unit, step4, tile4, step2, tile2, wave, serial, group;
     };
-    static constexpr Cost kSqrt{12, 1.0, 0.14, 0.28, 0.52, 6e-4, 0.060, 3.6e-4};
+    static constexpr Cost kSqrt{11, 0.82, 0.14, 0.13, 1.0, 5.4e-4, 0.053, 3.5e-4};
     static constexpr Cost kPow{6.5, 0.3, 0.58, 0.25, 0.30, 7.6e-4, 0.056, 4.5e-4};
     static constexpr Cost kSquare{9, 0.5, 0.06, 0.26, 0.09, 5.5e-4, 0.040, 2.7e-4};
     const Cost &c = fn == PT_SQRT ? kSqrt : fn == PT_SQUARE ? kSquare : kPow;
@@ -532,15 +533,17 @@ bool pt_direct_faster(int fn, long long rows, int rw, int N, int lag_first, int 
     const double n = N - (a < 0 && b > 0 ? (a * a + b * b) / (2 * (b - a)) : std::abs(a + b) / 2);
     // tiles
     const double windows = sp.ns > 1 ? 1.0 : (double)rw / sp.G, steps = n / 32 / sp.ns;
-    const int tiles = std::min((std::min(L, sp.lags) + 62) / 32, kPtWaves * tpw), deep = (tiles + kPtWaves - 1) / kPtWaves;
+    // tiles a wave of a lag block, on average: all of them but in the last one
+    const int last = L - (sp.nblk - 1) * 32 * pt_bands(tpw), tiles = std::min((last + 62) / 32, kPtWaves * tpw);
+    const double deep = (double)((sp.nblk - 1) * tpw + (tiles + kPtWaves - 1) / kPtWaves) / sp.nblk;
     const double rounds = (double)rows * sp.G * sp.nblk / (tpw == 4 ? 512 : 768);
     const double turns = rounds <= 1 ? 0.6 : rounds < 3 ? std::ceil(rounds) : rounds + 0.5;
     const double step = tpw == 4 ? c.step4 + c.tile4 * deep : c.step2 + c.tile2 * deep;
     const double tiled = turns * (c.unit + windows * steps * step);
-    // one lag a thread: four-norm of the two bounds
+    // one lag a thread: between the larger of the two bounds and their sum
     const double work = rw * n / 32 * rows * (c.wave * ((L + 63) / 64) + c.group * ((L + kPdLags - 1) / kPdLags));
     const double alone = rw * n * c.serial;
-    return std::sqrt(std::hypot(work * work, alone * alone)) < tiled;
+    return std::pow(std::pow(work, 2.5) + std::pow(alone, 2.5), 0.4) < tiled;
 }
 
 template <int TPW>

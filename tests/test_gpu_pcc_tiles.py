@@ -1,5 +1,5 @@
 """Time-domain PCC1 / PCC-v where the tiled kernel can go wrong: lag blocks of up to 224
-and 480 lags (bands of 32, equal blocks), chunks of 512 samples, split and unsplit
+and 480 lags (bands of 32), chunks of 512 samples, split and unsplit
 launches, and the records that decide between its two ways of summing PCC1's terms; and
 the kernel of one lag a thread at its edges."""
 import ctypes
