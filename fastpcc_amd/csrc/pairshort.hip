@@ -15,6 +15,7 @@
 // 248 us, 80 us; 97 stations x 17 x 2880 Gram 304 us, 284 us.  Bound by reading the
 // spectra through the caches.
 #include <algorithm>
+#include <type_traits>
 #include "edge.hpp"
 #include "engine.hpp"
 #include "kernels.hpp"
@@ -117,10 +118,15 @@ k_pair_short(PsArgs a, GnBatch jb)
     int i = 0, j = 0;
     if (SRC != PS_GRAM || a.edge) pair_index(p, a.S, i, j);
     // folded sums (see pcc2.hip): av at bin k, cv at M - k, ph at M/2
-    cf32 av[4], cv[4], ph = cf32{0.f, 0.f};
+    typedef std::conditional_t<SRC != PS_GRAM && MODE == 1, cf64, cf32> Acc;  // the windows' sums
+    Acc av[4], cv[4], ph{};
 #pragma unroll
-    for (int q = 0; q < 4; ++q) av[q] = cv[q] = cf32{0.f, 0.f};
-    if (SRC == PS_GRAM) {
+    for (int q = 0; q < 4; ++q) av[q] = cv[q] = Acc{};
+    auto add = [](Acc &s, cf32 v) {
+        s.x += v.x;
+        s.y += v.y;
+    };
+    if constexpr (SRC == PS_GRAM) {
         auto G = [&](int k) {
             return a.A[(long long)(k >> a.gl.sh) * a.gl.gs + p * a.gl.pl + (k & ((1 << a.gl.sh) - 1))];
         };
@@ -140,21 +146,21 @@ k_pair_short(PsArgs a, GnBatch jb)
                 const int k = t + NT * q;
                 const cf32 y0 = Y(k), y2 = Y(M - k);
                 if (SRC == PS_REAL) {
-                    av[q] = av[q] + y0;
-                    cv[q] = cv[q] + y2;
+                    add(av[q], y0);
+                    add(cv[q], y2);
                 } else {
                     const cf32 y1 = Y((Nz - k) & (Nz - 1)), y3 = Y(M + k);
-                    av[q] = av[q] + cf32{y0.x + y1.x, y0.y - y1.y};
-                    cv[q] = cv[q] + cf32{y2.x + y3.x, y2.y - y3.y};
+                    add(av[q], cf32{y0.x + y1.x, y0.y - y1.y});
+                    add(cv[q], cf32{y2.x + y3.x, y2.y - y3.y});
                 }
             }
             if (t == 0) {
                 const cf32 u0 = Y(M / 2);
                 if (SRC == PS_REAL) {
-                    ph = ph + u0;
+                    add(ph, u0);
                 } else {
                     const cf32 u1 = Y(Nz - M / 2);
-                    ph = ph + cf32{u0.x + u1.x, u0.y - u1.y};
+                    add(ph, cf32{u0.x + u1.x, u0.y - u1.y});
                 }
             }
         }
@@ -166,13 +172,13 @@ k_pair_short(PsArgs a, GnBatch jb)
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const int k = t + NT * q;
-        cf32 x = av[q], z = cv[q];
+        cf32 x = cf32{(float)av[q].x, (float)av[q].y}, z = cf32{(float)cv[q].x, (float)cv[q].y};
         if (k == 0) x.y = z.y = 0.f;  // DC and Nyquist of a real signal's spectrum are real
         const cf32 w = a.twc[k];
         buf0[k] = fold(x, z, w);
         if (k) buf0[M - k] = fold(z, x, cf32{-w.x, w.y});
     }
-    if (t == 0) buf0[M / 2] = cf32{2.f * ph.x, -2.f * ph.y};
+    if (t == 0) buf0[M / 2] = cf32{2.f * (float)ph.x, -2.f * (float)ph.y};
     __syncthreads();
     const cf32 *z = ps_ifft<M>(buf0, buf1, a.tw, t);
     if (!live) return;

@@ -1,0 +1,29 @@
+"""Errors against 64 bits that the FP32 stages are built to keep: 2-norm of the difference
+over 2-norm of the result, on records of noise with a common source."""
+import numpy as np
+import pytest
+
+from fastpcc_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def _error(fp, orc, kind, stack, S, W, N, lag1, lag2, x=None, **kw):
+    if x is None:
+        x, _ = synth.make_stations(S, W * N, 100, seed=N + S)
+    y = fp.allpairs(x, W, N, lag1, lag2, kind=kind, stack=stack, **kw).astype(np.float64)
+    r = orc.allpairs(kind, x, W, N, lag1, lag2, stacked=stack != "none", f64=True, **kw)
+    e = float(np.linalg.norm(y - r) / np.linalg.norm(r))
+    print(f"{kind}/{stack} S={S} W={W} N={N}: {e:.2e}", flush=True)
+    return e
+
+
+@pytest.mark.parametrize("N", [450, 900, 1800, 3600])
+def test_mean_of_many_windows(fp, orc, N):
+    """One source in every window: its spectra add up coherently, and a sum of 2000 of them
+    in FP32 would be off by 2^-25 sqrt(2000 / 3) = 8e-7 of itself; in FP64 what is left is
+    the inverse of nearly one value, under 2^-24."""
+    W = 2000
+    x = np.repeat(np.random.default_rng(N).standard_normal(W * N).astype(np.float32)[None], 2, axis=0)
+    x[1] += 0.3 * np.random.default_rng(1).standard_normal(W * N).astype(np.float32)
+    assert _error(fp, orc, "cc1b", "plain", 2, W, N, -50, 50, x=x) <= 2.0 ** -24
