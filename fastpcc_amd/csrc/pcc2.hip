@@ -52,12 +52,13 @@ __device__ void station_pcc_row(const float *__restrict__ in, int N, int Nz, con
     __syncthreads();
     cf32 *other = (X == buf0) ? buf1 : buf0;
     cf32 *z = fft_lds<float, +1>(X, other, planN, twN);
+    // the analytic signal's real part is the window itself: without the transforms' error.
     // AmpNormf (:178-205): eps = 1e-6*sqrt(max|z|^2) in double, stored as float
     float m = 0.0f;
     for (int n = threadIdx.x; n < N; n += T) {
-        cf32 v = z[n];
-        float a = v.x * v.x + v.y * v.y;
-        m = fmaxf(m, a);
+        const cf32 v = cf32{in[n], z[n].y};
+        z[n].x = v.x;
+        m = fmaxf(m, v.x * v.x + v.y * v.y);
     }
     m = block_max(m, red);
     const float eps = (float)(1e-6 * sqrt((double)m));
@@ -164,6 +165,12 @@ k_station_pcc_3600(const float *__restrict__ x, long long station_stride, int W,
     // samples b + 225 r (b < 225) of the analytic signal in registers
     ct_first_pass_regs<float, kSpN, kSpT, +1, 25, 0>(v, alt);
     ct_pass_oop<float, kSpN, kSpT, +1, 9, 25, 0, 0>(alt, lds, twI + 24);
+    // the real parts of those samples are the window itself, without the transforms' error
+    float xr[16];
+    if (t < kB) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) xr[r] = in[t + kB * r];
+    }
     ct_last_pass_regs<float, kSpN, kSpT, +1, 16, 0>(lds, v, twI + 24 + 8 * 25);
     // AmpNormf: max |z|^2 from registers; the samples go through alt (last read by
     // the inverse's second pass) to the 4096-point transforms' distribution, and
@@ -173,6 +180,7 @@ k_station_pcc_3600(const float *__restrict__ x, long long station_stride, int W,
     if (t < kB) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
+            v[r].x = xr[r];
             m = fmaxf(m, v[r].x * v[r].x + v[r].y * v[r].y);
             alt[t + kB * r] = v[r];
         }
