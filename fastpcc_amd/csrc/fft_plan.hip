@@ -258,13 +258,14 @@ const void *get_order_twiddles(int n, const std::vector<int> &radices, bool f64)
     return d;
 }
 
-const void *get_split_twiddles(int n)
+const void *get_split_twiddles(int n, bool f64)
 {
-    static std::map<std::pair<int, int>, const void *> cache;
+    static std::map<std::tuple<int, int, bool>, const void *> cache;
     int dev = 0;
     (void)hipGetDevice(&dev);
     std::lock_guard<std::mutex> lk(g_mu);
-    auto it = cache.find({dev, n});
+    const auto key = std::make_tuple(dev, n, f64);
+    auto it = cache.find(key);
     if (it != cache.end()) return it->second;
     if (!table_builds_allowed()) return nullptr;
     std::vector<double> t;
@@ -282,8 +283,8 @@ const void *get_split_twiddles(int n)
         t.push_back(c);
         t.push_back(s);
     }
-    const void *d = upload_table<float>(t);
-    cache.emplace(std::make_pair(dev, n), d);
+    const void *d = f64 ? upload_table<double>(t) : upload_table<float>(t);
+    cache.emplace(key, d);
     return d;
 }
 

@@ -16,6 +16,10 @@
 // its sums in the scratch row's own place; k_long_lags adds the shares and writes the
 // normalised lags.  Shares go to consecutive workgroups, so each XCD keeps reading
 // the same eighth (or quarter ..) of every station's spectrum, which its L2 holds.
+// Twiddles are products of FP64 table entries rounded once, and the shares are added in
+// FP64: with FP32 ones the fold and the sums cost more accuracy than the passes saved
+// (16 stations x 86400, 1-bit: error against 64 bits 1.90e-7 in two passes, 2.03e-7 with
+// FP32 twiddles, 1.78e-7 so; at most 3% of the time).
 // Against the inverse row and column passes (rows of Nz written and read again, both
 // of full length): 32 stations x 86400, +-2000 lags 477 -> 208 us, one pair x 649
 // windows x 21600, +-3000 lags 282 -> 165 us; bound by reading the spectra
@@ -39,7 +43,8 @@ struct LongArgs {
     long long bstride;
     int N1, S, W, Wb, wsel, wsum, pair0;  // as RowArgs
     int G, upg, A;              // shares an item, units a share, largest |n1|
-    const cf32 *twN, *twH, *twR, *twC;  // split table of Nz, passes of H, full tables of N1 and N2
+    const cf32 *twH, *twR;      // passes of H, full table of N1
+    const cf64 *twN, *twC;      // split table of Nz, full table of N2
 };
 
 __host__ __device__ constexpr int lp_ld(int H) { return H == 256 ? 274 : H == 512 ? 544 : 1088; }
@@ -51,6 +56,8 @@ __device__ __forceinline__ void lp_rows_ifft(cf32 *lds, const cf32 *__restrict__
     else if constexpr (H == 512) ctb_fft<512, 8, lp_ld(512), +1, 8, 8, 8>(lds, tw);
     else ctb_fft<1024, 4, lp_ld(1024), +1, 16, 8, 8>(lds, tw);
 }
+
+__device__ __forceinline__ cf32 lp_round(cf64 w) { return cf32{(float)w.x, (float)w.y}; }
 
 // Z[k] of the fold from a = Y[k] + conj Y[Nz-k] and c = Y[M-k] + conj Y[M+k], w = W_Nz^{-k}
 __device__ __forceinline__ cf32 lp_fold(cf32 a, cf32 c, cf32 w)
@@ -86,12 +93,11 @@ k_long_pair(LongArgs a)
         Fj = a.F2 + (long long)(cj * a.W + w0) * n;
     }
     const int pq = t / TP, c = t % TP;  // fold: row pair of the unit, first k2
-    const cf32 wc = conj(a.twC[c]);  // exp(2 pi i c / N2)
-    // sums: outputs n2 = t + 256 e; twiddles W_M^{k1 n2} and W_M^{N1 n2}
-    cf32 E[EP][AB + 1], O[EP][AB + 1], wH[EP];
+    const cf64 wc = conj(a.twC[c]);  // exp(2 pi i c / N2)
+    // sums: outputs n2 = t + 256 e
+    cf32 E[EP][AB + 1], O[EP][AB + 1];
 #pragma unroll
     for (int e = 0; e < EP; ++e) {
-        wH[e] = conj(a.twC[2 * (t + 256 * e)]);
 #pragma unroll
         for (int i = 0; i <= AB; ++i) E[e][i] = O[e][i] = cf32{0.f, 0.f};
     }
@@ -100,12 +106,12 @@ k_long_pair(LongArgs a)
             const int pi = u * PU + pq;  // row pair (pi, N1 - pi); (0, N1/2) for pi = 0
             const int ra = pi, rb = pi ? N1 - pi : N1 / 2;
             // row factor of the fold twiddles, exp(2 pi i pi / Nz) wc
-            const cf32 wr = cmul(conj(a.twN[pi]), wc);  // pi < kTwLo
+            const cf64 wr = cmul(conj(a.twN[pi]), wc);  // pi < kTwLo
             // four of a thread's eight bins at a time: their loads in flight together fill
             // the registers three workgroups a CU leave
 #pragma unroll 1
             for (int hs = 0; hs < 2; ++hs) {
-                const cf32 wrh = hs ? rot<+1>(wr) : wr;  // W_16^4 = i
+                const cf64 wrh = hs ? rot<+1>(wr) : wr;  // W_16^4 = i
                 const int k0 = c + 4 * TP * hs;
                 cf32 av[4], cv[4];
 #pragma unroll
@@ -134,7 +140,7 @@ k_long_pair(LongArgs a)
                 sfor<4>([&](auto sc) {
                     constexpr int s = sc();
                     const int k = k0 + TP * s;
-                    const cf32 w = twc<+1, 16, s>(wrh);  // exp(2 pi i TP s / N2) = W_16^s
+                    const cf32 w = lp_round(twc<+1, 16, s>(wrh));  // exp(2 pi i TP s / N2) = W_16^s
                     cf32 x = av[s], z = cv[s];
                     if (SRC == LP_REAL && pi == 0 && k == 0) x.y = z.y = 0.f;  // DC and Nyquist of a real signal
                     lds[pq * LD + ct_pad(k)] = lp_fold(x, z, w);
@@ -142,7 +148,7 @@ k_long_pair(LongArgs a)
                 });
             }
             if (pi == 0) {  // row N1/2: its own mirror, k2 -> N2 - 1 - k2
-                const cf32 wh = cmul(wr, conj(a.twN[N1 / 2]));
+                const cf64 wh = cmul(wr, conj(a.twN[N1 / 2]));
 #pragma unroll 1
                 for (int s = 0; s < 8; ++s) {
                     const int k = c + TP * s;
@@ -160,8 +166,7 @@ k_long_pair(LongArgs a)
                             z = z + cf32{y2.x + y3.x, y2.y - y3.y};
                         }
                     }
-                    const cf32 ws = conj(a.twC[TP * s]);
-                    lds[(PU + pq) * LD + ct_pad(k)] = lp_fold(x, z, cmul(wh, ws));
+                    lds[(PU + pq) * LD + ct_pad(k)] = lp_fold(x, z, lp_round(cmul(wh, conj(a.twC[TP * s]))));
                 }
             }
         }
@@ -175,13 +180,13 @@ k_long_pair(LongArgs a)
                 const int n2 = t + 256 * e;
                 const cf32 xa = lds[q * LD + ct_pad(n2)], xb = lds[(PU + q) * LD + ct_pad(n2)];
                 if (pi == 0) {  // rows 0 and N1/2: W^{(N1/2) n1} = (-1)^n1, W_M^{(N1/2) n2} = W_Nz^{N1 n2}
-                    const cf32 x1 = cmul(xb, conj(tw_m(a.twN, (unsigned)N1 * (unsigned)n2)));
+                    const cf32 x1 = cmul(xb, lp_round(conj(tw_m(a.twN, (unsigned)N1 * (unsigned)n2))));
                     const cf32 s = xa + x1, d = xa - x1;
 #pragma unroll
                     for (int i = 0; i <= AB; ++i) E[e][i] = E[e][i] + (i & 1 ? d : s);
                 } else {
-                    const cf32 wt = conj(tw_m(a.twN, 2u * (unsigned)pi * (unsigned)n2));
-                    const cf32 x0 = cmul(xa, wt), x1 = cmul(xb, cmulc(wt, wH[e]));
+                    const cf64 wt = conj(tw_m(a.twN, 2u * (unsigned)pi * (unsigned)n2));
+                    const cf32 x0 = cmul(xa, lp_round(wt)), x1 = cmul(xb, lp_round(conj(cmul(wt, a.twC[2 * n2]))));
                     const cf32 s = x0 + x1, d = x0 - x1;
 #pragma unroll
                     for (int i = 0; i <= AB; ++i) {
@@ -223,9 +228,9 @@ k_long_lags(ColArgs ca, const cf32 *__restrict__ C, long long bstride, int H, in
     if (ca.norm == 1) pair_index(p, ca.S, i, j);
     const int lag = ca.lag0 + l, m = lag >> 1;  // floor
     const float *row = reinterpret_cast<const float *>(C + (long long)b * bstride + (A * H + m)) + (lag & 1);
-    float v = 0.f;
-    for (int s = 0; s < G; ++s) v += row[2LL * s * gstride];
-    lagwin_store(ca, p, w, i, j, n, l, f * v);
+    double v = 0.0;
+    for (int s = 0; s < G; ++s) v += (double)row[2LL * s * gstride];
+    lagwin_store(ca, p, w, i, j, n, l, f * (float)v);
 }
 
 namespace {
@@ -294,12 +299,12 @@ int run_long_pair(const BigPlan &bp, const RowArgs &ra, const ColArgs &ca, bool 
     while ((2 * a.A + 1) * H > a.upg * 4096) a.upg *= 2;
     while (2 * a.upg <= U && (long long)nbatch * (U / (2 * a.upg)) >= 2048) a.upg *= 2;
     a.G = U / a.upg;
-    a.twN = bp.twN;
+    a.twN = (const cf64 *)get_split_twiddles(bp.n, true);
     a.twH = (const cf32 *)(H == 256 ? get_order_twiddles(256, {16, 16}) : H == 512 ? get_order_twiddles(512, {8, 8, 8})
                                                                           : get_order_twiddles(1024, {16, 8, 8}));
     a.twR = (const cf32 *)get_full_twiddles(bp.n1, false);
-    a.twC = (const cf32 *)get_full_twiddles(bp.n2, false);
-    if (!a.twH || !a.twR || !a.twC) return -1;
+    a.twC = (const cf64 *)get_full_twiddles(bp.n2, true);
+    if (!a.twN || !a.twH || !a.twR || !a.twC) return -1;
     if ((long long)nbatch * a.G > 0x7fffffff) return -1;
     const int src = gram ? LP_GRAM : real ? LP_REAL : LP_CROSS, blocks = nbatch * a.G, e = a.A * H / 256;
     int r;

@@ -7,7 +7,7 @@ namespace fpcc {
 
 // W_n^m from the two-factor table of get_split_twiddles (m < n): two small
 // cached lookups instead of a gather over an n-entry table
-__device__ __forceinline__ cf32 tw_m(const cf32 *__restrict__ twN, unsigned m)
+template <typename R> __device__ __forceinline__ C2<R> tw_m(const C2<R> *__restrict__ twN, unsigned m)
 {
     return cmul(twN[kTwLo + m / kTwLo], twN[m % kTwLo]);
 }
