@@ -189,7 +189,7 @@ struct PtSplit {
 template <int FN, int TPW>
 __global__ void __launch_bounds__(64 * kPtWaves) __attribute__((amdgpu_waves_per_eu(TPW == 4 ? 2 : 3)))
 k_pcc_time(const cf32 *__restrict__ phi, int S, int W, int N, int lag_first, int L, float V, double div, int mode,
-           PtSplit sp, float *__restrict__ y, int out_ld, int out_off, double *__restrict__ part)
+           PtSplit sp, int row0, float *__restrict__ y, int out_ld, int out_off, double *__restrict__ part)
 {
     constexpr int kT = 64 * kPtWaves, kTiles = kPtWaves * TPW, kA = kPtChunk + 32 * (kTiles - 1);
     __shared__ u4v bc[3][kPtChunk], ac[2][kA];                  // 2bx, 2by, -2by; ax, ay
@@ -200,7 +200,7 @@ k_pcc_time(const cf32 *__restrict__ phi, int S, int W, int N, int lag_first, int
     static_assert(sizeof(float) * kPtWaves * 32 * 33 <= sizeof(ac) && sizeof(double) * kTiles * 64 <= sizeof(bc), "fit");
     const int t = threadIdx.x, lane = t & 63, h = lane >> 5, lj = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int ru = blockIdx.x / sp.nblk, u = ru % sp.G, row = ru / sp.G;
+    const int ru = blockIdx.x / sp.nblk, u = ru % sp.G, row = row0 + ru / sp.G;
     // Workgroups go to the 8 XCDs in turn and the last lag block of a unit is short.  An even
     // number of blocks would put it on the same XCDs in every unit (780 pairs x 24 windows of
     // 1800, 481 lags: 8.7 ms, half the chip idle), so the blocks of a unit move on by one
@@ -412,12 +412,12 @@ __device__ __forceinline__ float pd_term(cf32 a, float ad, cf32 b, float bd, flo
 template <int FN>
 __global__ void __launch_bounds__(kPdLags)
 k_pcc_direct(const cf32 *__restrict__ phi, int S, int W, int N, int lag_first, int L, float V, double div, int mode,
-             int nblk, float *__restrict__ y, int out_ld, int out_off)
+             int nblk, int row0, float *__restrict__ y, int out_ld, int out_off)
 {
     constexpr int kA = kPdChunk + kPdLags;
     __shared__ cf32 sb[kPdChunk], sa[kA];    // 2 beta, alpha (0 outside the window)
     __shared__ float db[kPdChunk], da[kA];   // 1 - |.|^2
-    const int t = threadIdx.x, lb = blockIdx.x % nblk, row = blockIdx.x / nblk;
+    const int t = threadIdx.x, lb = blockIdx.x % nblk, row = row0 + blockIdx.x / nblk;
     const int p = mode == 0 ? row / W : row;
     const int w0 = mode == 0 ? row - p * W : 0, w1 = mode == 0 ? w0 + 1 : W;
     int i, j;
@@ -548,12 +548,12 @@ bool pt_direct_faster(int fn, long long rows, int rw, int N, int lag_first, int 
 
 template <int TPW>
 int launch_pt(int fn, const cf32 *d_phi, int S, int W, int N, int lag_first, int L, float V, double div, int mode,
-              const PtSplit &sp, long long blocks, float *d_y, int out_ld, int out_off, double *part, hipStream_t st)
+              const PtSplit &sp, int row0, unsigned blocks, float *d_y, int out_ld, int out_off, double *part, hipStream_t st)
 {
-    const dim3 g((unsigned)blocks), b(64 * kPtWaves);
+    const dim3 g(blocks), b(64 * kPtWaves);
 #define FPCC_PT(FN)                                                                                               \
-    hipLaunchKernelGGL((k_pcc_time<FN, TPW>), g, b, 0, st, d_phi, S, W, N, lag_first, L, V, div, mode, sp, d_y, out_ld, \
-                       out_off, part)
+    hipLaunchKernelGGL((k_pcc_time<FN, TPW>), g, b, 0, st, d_phi, S, W, N, lag_first, L, V, div, mode, sp, row0, d_y,    \
+                       out_ld, out_off, part)
     switch (fn) {
     case PT_SQRT: FPCC_PT(PT_SQRT); break;
     case PT_SQUARE: FPCC_PT(PT_SQUARE); break;
@@ -585,9 +585,8 @@ int launch_pcc_time(const cf32 *d_phi, int S, int W, int N, int lag_first, int L
     const int tpw = pt_tpw(rows, rw, L);
     PtSplit sp = pt_split(rows, rw, N, L, tpw);
     if (!part) sp.G = sp.ns = 1;
-    const long long blocks = rows * sp.G * sp.nblk;
-    if (blocks > 0x7fffffff) {
-        fprintf(stderr, "fastpcc: %lld lag blocks exceed one launch\n", blocks);
+    if (rows > 0x7fffffff) {
+        fprintf(stderr, "fastpcc: %lld output rows exceed one job\n", rows);
         return -1;
     }
     const float V = (float)(v / 2);
@@ -598,26 +597,34 @@ int launch_pcc_time(const cf32 *d_phi, int S, int W, int N, int lag_first, int L
     const double div = (pcc1 ? 2.0 : pow(2.0, (double)V)) * rw;
     const bool direct = fn == PT_POW || pt_direct_faster(fn, rows, rw, N, lag_first, L, tpw, sp);
     ProfScope prof(direct ? (pcc1 ? "pcc1_direct" : "pccv_direct") : pcc1 ? "pcc1_time" : "pccv_time", st);
-    int r;
-    if (direct) {
-        const int nblk = (L + kPdLags - 1) / kPdLags;
-        if (rows * nblk > 0x7fffffff) return -1;
-        const dim3 g((unsigned)(rows * nblk)), b(kPdLags);
+    // a launch holds fewer than 2^32 threads (more wrap around unnoticed): the rows of one
+    // launch at a time; rows that are split (G > 1) are few
+    constexpr long long kMostBlocks = 1 << 23;
+    const int nblk = direct ? (L + kPdLags - 1) / kPdLags : sp.nblk, G = direct ? 1 : sp.G;
+    const long long step = std::max(1LL, kMostBlocks / ((long long)nblk * G));
+    for (long long r0 = 0; r0 < rows; r0 += step) {
+        const int row0 = (int)r0;
+        const unsigned blocks = (unsigned)(std::min(step, rows - r0) * G * nblk);
+        if (direct) {
+            const dim3 g(blocks), b(kPdLags);
 #define FPCC_PD(FN)                                                                                               \
-    hipLaunchKernelGGL(k_pcc_direct<FN>, g, b, 0, st, d_phi, S, W, N, lag_first, L, V, div, mode, nblk, d_y, out_ld, out_off)
-        switch (fn) {
-        case PT_SQRT: FPCC_PD(PT_SQRT); break;
-        case PT_SQUARE: FPCC_PD(PT_SQUARE); break;
-        case PT_HWPOW: FPCC_PD(PT_HWPOW); break;
-        default: FPCC_PD(PT_POW); break;
-        }
+    hipLaunchKernelGGL(k_pcc_direct<FN>, g, b, 0, st, d_phi, S, W, N, lag_first, L, V, div, mode, nblk, row0, d_y,    \
+                       out_ld, out_off)
+            switch (fn) {
+            case PT_SQRT: FPCC_PD(PT_SQRT); break;
+            case PT_SQUARE: FPCC_PD(PT_SQUARE); break;
+            case PT_HWPOW: FPCC_PD(PT_HWPOW); break;
+            default: FPCC_PD(PT_POW); break;
+            }
 #undef FPCC_PD
-        FPCC_CHECK(hipGetLastError());
-        return 0;
+            FPCC_CHECK(hipGetLastError());
+            continue;
+        }
+        const auto launch = tpw == 4 ? launch_pt<4> : launch_pt<2>;
+        const int r = launch(fn, d_phi, S, W, N, lag_first, L, V, div, mode, sp, row0, blocks, d_y, out_ld, out_off, part, st);
+        if (r) return r;
     }
-    if (tpw == 4) r = launch_pt<4>(fn, d_phi, S, W, N, lag_first, L, V, div, mode, sp, blocks, d_y, out_ld, out_off, part, st);
-    else r = launch_pt<2>(fn, d_phi, S, W, N, lag_first, L, V, div, mode, sp, blocks, d_y, out_ld, out_off, part, st);
-    if (r || sp.G == 1) return r;
+    if (G == 1) return 0;
     hipLaunchKernelGGL(k_pcc_time_sum, dim3((L + 255) / 256, (unsigned)rows), dim3(256), 0, st, part, N, lag_first, L,
                        sp.G, div, d_y, out_ld, out_off);
     FPCC_CHECK(hipGetLastError());

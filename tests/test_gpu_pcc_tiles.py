@@ -186,3 +186,19 @@ def test_host_entry_at_a_negative_power(fp):
     y = fp.pcc_set(*x.reshape(2, W, N), v, -30, 200)
     assert np.isfinite(y).all()
     assert np.array_equal(y, fp.allpairs(x, W, N, -30, 200, kind="pccv", stack="none", v=v)[0])
+
+
+# more than 2^32 threads: the rows of one launch at a time
+@pytest.mark.parametrize("kind,lag1,lag2", [("pcc1", 0, 0), ("pccv", -2, 1)])
+def test_more_rows_than_one_launch(fp, kind, lag1, lag2):
+    S, W, N = 2000, 10, 8
+    x = np.random.default_rng(2).standard_normal((S, W * N)).astype(np.float32)
+    y = fp.allpairs(x, W, N, lag1, lag2, kind=kind, stack="none", v=1.5)
+    # the pairs of the first three and of the last four stations
+    first = fp.allpairs(x[:3], W, N, lag1, lag2, kind=kind, stack="none", v=1.5)
+    last = fp.allpairs(x[-4:], W, N, lag1, lag2, kind=kind, stack="none", v=1.5)
+    tol = 2.0 ** -22  # FP32 terms summed in another order
+    assert np.abs(y[[0, 1, S - 1]] - first).max() <= tol and np.abs(y[-6:] - last).max() <= tol
+    # every row is written: a correlation of 6 and more noise samples is not exactly 0
+    assert (np.abs(y).max(axis=-1) > 0).all()
+
