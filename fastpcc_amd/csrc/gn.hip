@@ -135,10 +135,10 @@ __global__ void __launch_bounds__(512)
 k_pair_gn(const C2<T> *__restrict__ Xa, const C2<T> *__restrict__ Xb, long long ldx,
           const double *__restrict__ E, long long lde, int S, int W, int N, int Nz, FftPlan planM,
           const C2<T> *__restrict__ twM, const C2<T> *__restrict__ twc, int lag0, int L, int norm, int mode,
-          float *__restrict__ y, const float *__restrict__ edge, int K, GnBatch jb)
+          float *__restrict__ y, const float *__restrict__ edge, int K, GnBatch jb, int block0)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    int bid = blockIdx.x;
+    int bid = blockIdx.x + block0;
     if (BATCH) {
         int jj = 0;
         while (jj + 1 < jb.n && bid >= jb.b0[jj + 1]) ++jj;
@@ -354,8 +354,9 @@ int launch_pair_gn(const void *d_Xa, const void *d_Xb, const double *d_E, bool f
     const void *twc = get_c2r_twiddles(Nz, f64);
     if (!pM.ok || !twc) return -1;
     const int P = S * (S - 1) / 2;
-    const int blocks = mode == 0 ? P * W : P;
+    const long long blocks = mode == 0 ? (long long)P * W : P;
     if (!blocks) return 0;
+    if (blocks > 0x7fffffff) return -1;
     const size_t elem = f64 ? sizeof(cf64) : sizeof(cf32);
     // Nz 8192: the compile-time in-place inverse and its own twiddle order
     const bool ct = f64 && M == 4096;
@@ -370,15 +371,17 @@ int launch_pair_gn(const void *d_Xa, const void *d_Xb, const double *d_E, bool f
     if (f64) {
         const auto fn = ct ? k_pair_gn<double, true, false> : k_pair_gn<double, false, false>;
         allow_lds((const void *)fn, lds);
-        hipLaunchKernelGGL(fn, dim3(blocks), dim3(512), lds, st, (const cf64 *)d_Xa, (const cf64 *)d_Xb,
-                           real_ld(Nz), d_E, energy_ld(N), S, W, N, Nz, pM.plan, (const cf64 *)tw,
-                           (const cf64 *)twc, lag0, L, norm, mode, d_y, d_edge, K, GnBatch{});
+        for (long long b = 0; b < blocks; b += kMostBlocks)
+            hipLaunchKernelGGL(fn, dim3((unsigned)std::min(kMostBlocks, blocks - b)), dim3(512), lds, st,
+                               (const cf64 *)d_Xa, (const cf64 *)d_Xb, real_ld(Nz), d_E, energy_ld(N), S, W, N, Nz, pM.plan,
+                               (const cf64 *)tw, (const cf64 *)twc, lag0, L, norm, mode, d_y, d_edge, K, GnBatch{}, (int)b);
     } else {
         const auto fn = k_pair_gn<float, false, false>;
         allow_lds((const void *)fn, lds);
-        hipLaunchKernelGGL(fn, dim3(blocks), dim3(512), lds, st, (const cf32 *)d_Xa, (const cf32 *)d_Xb,
-                           real_ld(Nz), d_E, energy_ld(N), S, W, N, Nz, pM.plan, (const cf32 *)tw,
-                           (const cf32 *)twc, lag0, L, norm, mode, d_y, d_edge, K, GnBatch{});
+        for (long long b = 0; b < blocks; b += kMostBlocks)
+            hipLaunchKernelGGL(fn, dim3((unsigned)std::min(kMostBlocks, blocks - b)), dim3(512), lds, st,
+                               (const cf32 *)d_Xa, (const cf32 *)d_Xb, real_ld(Nz), d_E, energy_ld(N), S, W, N, Nz, pM.plan,
+                               (const cf32 *)tw, (const cf32 *)twc, lag0, L, norm, mode, d_y, d_edge, K, GnBatch{}, (int)b);
     }
     FPCC_CHECK(hipGetLastError());
     return 0;
@@ -416,17 +419,19 @@ int launch_pair_gn_batch(GnBatch jb, bool f64, int Nz, int norm, int mode, hipSt
     if (f64) {
         const auto fn = ct ? k_pair_gn<double, true, true> : k_pair_gn<double, false, true>;
         allow_lds((const void *)fn, lds);
-        hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(512), lds, st, (const cf64 *)nullptr,
-                           (const cf64 *)nullptr, real_ld(Nz), (const double *)nullptr, 0LL, 0, 0, 0, Nz, pM.plan,
-                           (const cf64 *)tw, (const cf64 *)twc, 0, 0, norm, mode, (float *)nullptr,
-                           (const float *)nullptr, 0, jb);
+        for (long long b = 0; b < blocks; b += kMostBlocks)
+            hipLaunchKernelGGL(fn, dim3((unsigned)std::min(kMostBlocks, blocks - b)), dim3(512), lds, st,
+                               (const cf64 *)nullptr, (const cf64 *)nullptr, real_ld(Nz), (const double *)nullptr, 0LL, 0, 0, 0,
+                               Nz, pM.plan, (const cf64 *)tw, (const cf64 *)twc, 0, 0, norm, mode, (float *)nullptr,
+                               (const float *)nullptr, 0, jb, (int)b);
     } else {
         const auto fn = k_pair_gn<float, false, true>;
         allow_lds((const void *)fn, lds);
-        hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(512), lds, st, (const cf32 *)nullptr,
-                           (const cf32 *)nullptr, real_ld(Nz), (const double *)nullptr, 0LL, 0, 0, 0, Nz, pM.plan,
-                           (const cf32 *)tw, (const cf32 *)twc, 0, 0, norm, mode, (float *)nullptr,
-                           (const float *)nullptr, 0, jb);
+        for (long long b = 0; b < blocks; b += kMostBlocks)
+            hipLaunchKernelGGL(fn, dim3((unsigned)std::min(kMostBlocks, blocks - b)), dim3(512), lds, st,
+                               (const cf32 *)nullptr, (const cf32 *)nullptr, real_ld(Nz), (const double *)nullptr, 0LL, 0, 0, 0,
+                               Nz, pM.plan, (const cf32 *)tw, (const cf32 *)twc, 0, 0, norm, mode, (float *)nullptr,
+                               (const float *)nullptr, 0, jb, (int)b);
     }
     FPCC_CHECK(hipGetLastError());
     return 0;

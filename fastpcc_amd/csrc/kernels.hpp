@@ -6,6 +6,10 @@
 
 namespace fpcc {
 
+// A launch holds fewer than 2^32 threads (more wrap around unnoticed): pair stages of one
+// workgroup or more a pair-window launch this many at a time.
+constexpr long long kMostBlocks = 1 << 22;
+
 // PCC2 station stage: F[s*W+w][Nz] = FFT_Nz(pad(AmpNormf(analytic_N(x_sw))))
 int launch_station_pcc(const float *d_x, long long station_stride, int S, int W, int N, int Nz, cf32 *d_F,
                        hipStream_t st);

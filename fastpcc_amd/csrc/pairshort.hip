@@ -88,13 +88,13 @@ __device__ __forceinline__ cf32 *ps_ifft(cf32 *a, cf32 *b, const cf32 *__restric
 // MODE 0: every window, y[p][w][L]; 1: the windows' mean (Gram rows: already summed)
 template <int M, int SRC, int MODE, bool BATCH>
 __global__ void __launch_bounds__(M == 4096 ? 512 : 256)
-k_pair_short(PsArgs a, GnBatch jb)
+k_pair_short(PsArgs a, GnBatch jb, int block0)
 {
     constexpr int NT = M / 8, TB = M == 4096 ? 512 : 256, TPB = TB / NT, Nz = 2 * M;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int g = threadIdx.x / NT, t = threadIdx.x % NT;
     cf32 *buf0 = reinterpret_cast<cf32 *>(smem_raw) + g * 2 * M, *buf1 = buf0 + M;
-    const int unit = blockIdx.x * TPB + g;
+    const int unit = (blockIdx.x + block0) * TPB + g;
     const bool live = unit < a.units;
     int u = live ? unit : a.units - 1;
     if (BATCH) {
@@ -208,8 +208,10 @@ int launch_ps_t(const PsArgs &a, const GnBatch &jb, hipStream_t st)
 {
     constexpr int NT = M / 8, TB = M == 4096 ? 512 : 256, TPB = TB / NT;
     const size_t lds = sizeof(cf32) * 2 * M * TPB;
-    hipLaunchKernelGGL((k_pair_short<M, SRC, MODE, BATCH>), dim3((unsigned)((a.units + TPB - 1) / TPB)), dim3(TB), lds, st, a,
-                       jb);
+    const long long blocks = ((long long)a.units + TPB - 1) / TPB;
+    for (long long b = 0; b < blocks; b += kMostBlocks)
+        hipLaunchKernelGGL((k_pair_short<M, SRC, MODE, BATCH>), dim3((unsigned)std::min(kMostBlocks, blocks - b)), dim3(TB), lds,
+                           st, a, jb, (int)b);
     FPCC_CHECK(hipGetLastError());
     return 0;
 }

@@ -290,7 +290,7 @@ __device__ __forceinline__ float real_out(const cf32 *z, int n)
 __global__ void __launch_bounds__(512)
 k_pair_pcc2(const cf32 *__restrict__ F, int S, int W, int Nz, FftPlan planM, const cf32 *__restrict__ twM,
             const cf32 *__restrict__ twc, int lag0, int L, float scale, int mode,
-            float *__restrict__ y)
+            int block0, float *__restrict__ y)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int M = Nz >> 1;
@@ -298,11 +298,11 @@ k_pair_pcc2(const cf32 *__restrict__ F, int S, int W, int Nz, FftPlan planM, con
     cf32 *buf1 = buf0 + M;
     int p, w0, w1;
     if (mode == 0) {
-        p = blockIdx.x / W;
-        w0 = blockIdx.x % W;
+        p = (blockIdx.x + block0) / W;
+        w0 = (blockIdx.x + block0) % W;
         w1 = w0 + 1;
     } else {
-        p = blockIdx.x;
+        p = blockIdx.x + block0;
         w0 = 0;
         w1 = W;
     }
@@ -434,11 +434,13 @@ int launch_pair_pcc2(const cf32 *d_F, int S, int W, int N, int Nz, int lag0, int
     const float scale = 1 / ((float)Nz * (float)N);
     const int threads = 512;
     const size_t lds = sizeof(cf32) * 2 * (size_t)M;
-    int blocks = mode == 0 ? npairs * W : npairs;
+    const long long blocks = mode == 0 ? (long long)npairs * W : npairs;
     if (blocks == 0) return 0;
+    if (blocks > 0x7fffffff) return -1;
     ProfScope prof(mode ? "pair_pcc2_mean" : "pair_pcc2_none", st);
-    hipLaunchKernelGGL(k_pair_pcc2, dim3(blocks), dim3(threads), lds, st, d_F, S, W, Nz, pM.plan,
-                       (const cf32 *)pM.tw, (const cf32 *)twc, lag0, L, scale, mode, d_y);
+    for (long long b = 0; b < blocks; b += kMostBlocks)
+        hipLaunchKernelGGL(k_pair_pcc2, dim3((unsigned)std::min(kMostBlocks, blocks - b)), dim3(threads), lds, st, d_F, S, W,
+                           Nz, pM.plan, (const cf32 *)pM.tw, (const cf32 *)twc, lag0, L, scale, mode, (int)b, d_y);
     FPCC_CHECK(hipGetLastError());
     return 0;
 }

@@ -597,9 +597,7 @@ int launch_pcc_time(const cf32 *d_phi, int S, int W, int N, int lag_first, int L
     const double div = (pcc1 ? 2.0 : pow(2.0, (double)V)) * rw;
     const bool direct = fn == PT_POW || pt_direct_faster(fn, rows, rw, N, lag_first, L, tpw, sp);
     ProfScope prof(direct ? (pcc1 ? "pcc1_direct" : "pccv_direct") : pcc1 ? "pcc1_time" : "pccv_time", st);
-    // a launch holds fewer than 2^32 threads (more wrap around unnoticed): the rows of one
-    // launch at a time; rows that are split (G > 1) are few
-    constexpr long long kMostBlocks = 1 << 23;
+    // the rows of one launch at a time; rows that are split (G > 1) are few
     const int nblk = direct ? (L + kPdLags - 1) / kPdLags : sp.nblk, G = direct ? 1 : sp.G;
     const long long step = std::max(1LL, kMostBlocks / ((long long)nblk * G));
     for (long long r0 = 0; r0 < rows; r0 += step) {

@@ -48,3 +48,15 @@ def test_windows_over_the_chip(fp, orc, S, W, stack):
 def test_one_sided(fp, orc):
     _check(fp, orc, "pcc2", "none", 5, 2, 1500, 37, 38)
     _check(fp, orc, "cc1b", "plain", 5, 2, 1500, -1400, -1399)
+
+
+@pytest.mark.parametrize("kind", ["pcc2", "gncc", "cc1b"])
+def test_more_pair_windows_than_one_launch(fp, kind):
+    """20 million pair-windows, a workgroup of 512 threads each: more than 2^32 threads."""
+    S, W, N = 2000, 10, 8
+    x = np.random.default_rng(2).standard_normal((S, W * N)).astype(np.float32)
+    y = fp.allpairs(x, W, N, -1, 2, kind=kind, stack="none")
+    first, last = (fp.allpairs(v, W, N, -1, 2, kind=kind, stack="none") for v in (x[:3], x[-4:]))
+    assert np.array_equal(y[[0, 1, S - 1]], first) and np.array_equal(y[-6:], last)
+    if kind != "cc1b":  # 6 and more samples of noise: never 0 at every lag
+        assert (np.abs(y).max(axis=-1) > 0).all()
