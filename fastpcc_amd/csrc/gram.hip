@@ -943,7 +943,8 @@ k_pair_c2r_4096(const cf32 *__restrict__ G, GLayout gl, int P, const cf32 *__res
     }
 }
 
-// The per pair-window PCC2 pair stage for Nz = 8192 on the same transform.
+// The PCC2 pair stage without a Gram (every window, or summed over the windows) for
+// Nz = 8192 on the same transform.
 // Persistent workgroups walk the pairs; for each window w of pair (i, j) thread t
 // forms, for its bins k = t + NT q (k < M/2) and their mirrors M - k, the folded
 // cross spectrum Gf(k) = Y(k) + conj Y(Nz-k), Y = conj(F_i,w) F_j,w, from the bins
@@ -1326,7 +1327,7 @@ static int launch_c2r_4096(const cf32 *d_G, const GLayout &gl, int P, const cf32
 
 // Workgroups of the pair kernel that run at once, and the units a pair's windows are
 // split into when the pairs alone (MODE 0) do not fill them: one pair of 24 windows took
-// 119 us on one workgroup, 11 us on 24.
+// 119 us on one workgroup, 10 us on 24.
 template <int MODE, bool ENDS, bool BATCH>
 static int launch_plain_4096_t(const cf32 *d_F, int S, int W, int P, const int *order, const cf32 *twr, const cf32 *twc,
                                int lag0, int L, float scale, float *d_y, const PlainBatch &jb, hipStream_t st,

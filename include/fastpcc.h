@@ -121,7 +121,7 @@ int cuda_tspcc2_set_freq(float **y0, float **x01, float **x02, unsigned int N, u
  * the arithmetic mean over windows.  Stack modes per kind: PCC2 all; GNCC NONE,
  * PLAIN (its per-window energies forbid stacking spectra); 1-bit NONE, PLAIN, GRAM,
  * GRAM16;
- * PCC1 and PCC-v NONE, PLAIN (time-domain sums, N <= 8192); WPCC NONE, PLAIN
+ * PCC1 and PCC-v NONE, PLAIN (time-domain sums); WPCC NONE, PLAIN
  * (= GRAM: the sum over scales and windows is one per-frequency Gram).
  *
  * FPCC_STACK_PWS (PCC2, GNCC and 1-bit, zero-pad length Nz <= 8192): the
@@ -137,8 +137,10 @@ int cuda_tspcc2_set_freq(float **y0, float **x01, float **x02, unsigned int N, u
 enum { FPCC_PCC2 = 0, FPCC_PCC1 = 1, FPCC_PCCV = 2, FPCC_GNCC = 3, FPCC_CC1B = 4, FPCC_WPCC = 5 };
 enum {
     FPCC_STACK_NONE = 0,  /* per-window outputs                                       */
-    FPCC_STACK_PLAIN = 1, /* mean of per-window correlations (PCC2 and 1-bit: one IFFT of the summed spectra) */
-    FPCC_STACK_ZSUM = 2,  /* sum of folded cross spectra over windows, one IFFT per pair */
+    FPCC_STACK_PLAIN = 1, /* mean of per-window correlations (PCC2 and 1-bit: one IFFT of the summed spectra;
+                           * GNCC, PCC1, PCC-v: window by window)                      */
+    FPCC_STACK_ZSUM = 2,  /* PCC2: the same sum of folded cross spectra over windows, one IFFT per pair (the
+                           * computation of PLAIN) */
     FPCC_STACK_GRAM = 3,  /* per-frequency Hermitian rank-W Gram (FP32 MFMA), one IFFT per pair */
     FPCC_STACK_GRAM16 = 4, /* the same Gram on FP16 MFMA with split hi+lo operands           */
     FPCC_STACK_PWS = 5     /* phase-weighted stack of the per-window correlations (below)    */
@@ -164,7 +166,11 @@ typedef struct {
 size_t fpcc_output_len(const fpcc_job *job);
 /* Device workspace bytes for a job (PCC1 and PCC-v of few pairs include a scratch of
  * at most some MB that spreads their sums over the chip; they also run without it,
- * more slowly, in the n_stations * n_windows * win_len phasors of 8 bytes alone). */
+ * more slowly, in the n_stations * n_windows * win_len phasors of 8 bytes alone).
+ * One job gives the same bits every time.  The same pair in jobs of another size, or
+ * PCC1 / PCC-v without the scratch, may differ in the last digits: the number of
+ * pairs, windows and lags decides the order of the FP32 and FP64 sums (long windows,
+ * means, time-domain sums). */
 size_t fpcc_workspace_size(const fpcc_job *job);
 /* Device buffers, stream-ordered on `stream` (a hipStream_t, NULL = default
  * stream); no allocation, no synchronisation.  Returns 0 or an error code. */
