@@ -434,7 +434,7 @@ k_big_cols(ColArgs a, int N1, int N2, FftPlan p1, const cf32 *__restrict__ tw1, 
 // else inverse, AmpNorm, forward, step twiddles, in place.  Reading the rows twice and
 // writing them once, against write + read of the analytic scales in between: 24
 // stations x 56 scales x 131072, 672 + 832 us as COL_INV_MAX and COL_FWD_AMPNORM of
-// k_big_cols, here 329 + 728 us (in k_big_cols itself the second transform took its
+// k_big_cols, here 328 + 723 us (in k_big_cols itself the second transform took its
 // registers from 167 to 213, and both passes lost: 772 + 1077 us).
 template <bool BATCH, bool MAX>
 __global__ void __launch_bounds__(256)

@@ -21,9 +21,9 @@
 // (16 stations x 86400, 1-bit: error against 64 bits 1.90e-7 in two passes, 2.03e-7 with
 // FP32 twiddles, 1.78e-7 so; at most 3% of the time).
 // Against the inverse row and column passes (rows of Nz written and read again, both
-// of full length): 32 stations x 86400, +-2000 lags 477 -> 208 us, one pair x 649
-// windows x 21600, +-3000 lags 282 -> 165 us; bound by reading the spectra
-// through the caches and by the folds.
+// of full length): 32 stations x 86400, +-2000 lags 477 -> 214 us, one pair x 649
+// windows x 21600, +-3000 lags 282 -> 167 us; bound by the latency of its loads and folds
+// (vector unit 21-30% busy, 1.7 TB/s of HBM).
 #include <algorithm>
 #include <cstdlib>
 #include "bigfft.hpp"

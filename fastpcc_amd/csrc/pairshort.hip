@@ -7,12 +7,12 @@
 // them: 32 KB, so that a CU holds several workgroups at every length.  Thread t folds
 // bins k = t + i M/8 (i < 4) and M - k from one load of each.  Where every window counts
 // alike (PCC2 and 1-bit: the overlap normalisation does not depend on the window) the mean
-// over windows is one inverse of the summed spectra; per-window outputs are a transform
+// over windows is one inverse of the spectra's sum (in FP64); per-window outputs are a transform
 // each, spread over the chip however few the pairs.
 // Whole jobs, against the runtime plan with 512 threads a transform and an inverse per
-// window: 45 stations x 30 windows of 1800, 1-bit, every window 526 us, here 259 us
-// (output 142 MB), their mean 459 us, 133 us; 50 stations x 20 x 600 PCC2, every window
-// 248 us, 80 us; 97 stations x 17 x 2880 Gram 304 us, 284 us.  Bound by reading the
+// window: 45 stations x 30 windows of 1800, 1-bit, every window 526 us, here 240 us
+// (output 142 MB), their mean 459 us, 135 us; 50 stations x 20 x 600 PCC2, every window
+// 248 us, 84 us; 97 stations x 17 x 2880 Gram 312 us, 291 us.  Bound by reading the
 // spectra through the caches.
 #include <algorithm>
 #include <type_traits>

@@ -23,10 +23,10 @@
 // of a term (|a+b| <= 2), throughout the wave, with a bound of |d| over the group's
 // rows; only groups that fail take the roots.  d is the difference of two
 // regularisers 1e-6 max|z| / |z|: 1e-5 in noise, where 1 in 10 groups fails; windows
-// with an event 30 times the noise fail mostly and run no slower than the roots alone.
+// with an event 30 times the noise fail mostly and take the roots as well.
 // 16 stations x 24 windows of 3600, 2001 lags: 9.40 ms with 12 vector operations a term
 // (sums, differences and squares formed term by term), 5.21 ms here, bound by the
-// vector unit (84% busy, about 7 operations a term).
+// vector unit (83% busy, 6.8 operations a term).
 #include <algorithm>
 #include "engine.hpp"
 #include "kernels.hpp"
