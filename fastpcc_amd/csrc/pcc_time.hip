@@ -515,7 +515,7 @@ PtSplit pt_split(long long rows, int rw, int N, int L, int tpw)
 // that hold lags; a chip they do not fill runs them faster.  One lag a thread: the
 // vector work of its waves, or a lone wave's latency.  The constants are those that pick
 // the faster one in 240 measured launches (S 2 .. 100, W 1 .. 30, N 16 .. 4096, up to 2001
-// lags; at worst 1.3x of the faster one's time, where the two are near each other and the
+// lags; at worst 1.15x of the faster one's time, where the two are near each other and the
 // records decide how many roots the tiles take).  The tiles alone ran at 0.1x of this
 // kernel's speed for 18720 windows of 16, 0.65 .. 0.85x for as many of 600 .. 2000 and up
 // to 501 lags; this kernel at 0.1x of theirs for few long windows.
@@ -540,9 +540,10 @@ bool pt_direct_faster(int fn, long long rows, int rw, int N, int lag_first, int 
     const double turns = rounds <= 1 ? 0.6 : rounds < 3 ? std::ceil(rounds) : rounds + 0.5;
     const double step = tpw == 4 ? c.step4 + c.tile4 * deep : c.step2 + c.tile2 * deep;
     const double tiled = turns * (c.unit + windows * steps * step);
-    // one lag a thread: between the larger of the two bounds and their sum
+    // one lag a thread: between the larger of the two bounds (the longest lag's, for one wave)
+    // and their sum
     const double work = rw * n / 32 * rows * (c.wave * ((L + 63) / 64) + c.group * ((L + kPdLags - 1) / kPdLags));
-    const double alone = rw * n * c.serial;
+    const double alone = rw * (N - (a < 0 && b > 0 ? 0.0 : std::min(std::abs(a), std::abs(b)))) * c.serial;
     return std::pow(std::pow(work, 2.5) + std::pow(alone, 2.5), 0.4) < tiled;
 }
 
